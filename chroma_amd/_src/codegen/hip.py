@@ -90,6 +90,19 @@ MID_GEMMS = True
 PREFETCH_WEIGHT_BYTES = (4 << 20, 64 << 20)
 PREFETCH_BLOCKS = 2048
 WEIGHT_PREFETCH = True
+# The K-split body (chroma::kwave_linear, KWAVE_WAVES waves a workgroup, each over its own share of K): the microseconds
+# of a launch are about KWAVE_OVERHEAD_US plus, per round of the chip's compute units, the larger of its tiles' operand
+# bytes at KWAVE_LOAD_GBS and their products at KWAVE_MATRIX_GFLOPS per unit. Measured over 12 bfloat16 and 9 float shapes
+# (rows 18-1000, columns 160-11520, K 128-11520, cold weights), with the larger figures for larger tiles: 41-55 GB/s.
+KWAVE_WAVES = 4
+KWAVE_OVERHEAD_US = 5.0
+KWAVE_LOAD_GBS = 53.0
+KWAVE_MATRIX_GFLOPS = {torch.float32: 480.0, torch.bfloat16: 5000.0}
+KWAVE_PREFETCH = (512, 8 << 20)  # rows from which, and weight bytes up to which, its weights are still read ahead
+KWAVE_LDS = 147 << 10  # bytes of LDS a workgroup's rings take at most
+# The tiled bodies by the same account: (rows, columns) of a tile, and the load rate they reach when every compute unit
+# has a tile (600 x 2880 x 4096 on 128 x 192 57 us, 700 x 11520 x 2880 89 us; 2048 x 5120 x 2880 on 256 x 192 66-82 us).
+TILED_LOAD_GBS = {(256, 192): 36.0, (128, 192): 44.0}
 # bfloat16 expert products whose channel count is a multiple of a tile width here (the first that fits)
 # take the ring body (chroma::grouped_expert_linear PATH 3) on 128-slot x width tiles with that many waves
 # side by side (each wave all slots of a width / waves strip), and an expert's last tile holds up to the
@@ -1971,7 +1984,7 @@ class HIPCodegen(Codegen):
             return out
         x = self.contiguous(x)
         inputs = [x, weight] + ([bias] if bias is not None else [])
-        if self.blas and rows <= 16 and inner % 4 == 0:
+        if self.blas and rows <= 16 and inner % 4 == 0 and not self._kwave_fits(x, weight, rows, columns, inner):
             self._skinny_linear(out, x, weight, bias, rows, columns, inner)
             self.skinny_matmuls += 1
         elif (self.blas and columns <= NARROW_COLUMNS and rows >= 64 and inner % (32 if meta.dtype == torch.bfloat16 else 4) == 0
@@ -2124,7 +2137,57 @@ class HIPCodegen(Codegen):
         self.launch(k, min(-(-size // (16 * 256)), PREFETCH_BLOCKS), 256, [weight], kind="prefetch")
         self.weight_prefetches += 1
 
+    @staticmethod
+    def _kwave_fits(x: Value, weight: Value, rows: int, columns: int, inner: int) -> bool:
+        """The K-split body applies: 16-byte aligned addresses and rows, byte offsets below 2^31, and a 64-byte unit of
+        K for every wave (with less, some waves have nothing to do and the sliced bodies' one or two slices are as
+        quick)."""
+        chunk, size = 16 // ITEMSIZE[x.dtype], ITEMSIZE[x.dtype]
+        return (inner % chunk == 0 and inner * size >= 64 * KWAVE_WAVES and x.view.offset % chunk == 0 and weight.view.offset % chunk == 0
+                and max(rows, 128) * inner * size < 2**31)
+
+    @staticmethod
+    def _kwave_plan(rows: int, columns: int, inner: int, dtype: torch.dtype) -> Tuple[float, int, int]:
+        """(estimated microseconds, 16-row blocks, 16-column blocks) of the K-split body's best tile: the account at
+        ``KWAVE_OVERHEAD_US`` over the tiles its registers and LDS allow (larger tiles move fewer operand bytes but
+        leave compute units idle once there are fewer tiles than units)."""
+        size, best = ITEMSIZE[dtype], None
+        for tm in range(1, min(8, -(-rows // 16)) + 1):
+            for tn in (1, 2, 3, 4, 6):
+                if tm * tn > 36 or 3 * KWAVE_WAVES * (tm + tn) << 10 > KWAVE_LDS:
+                    continue
+                rounds = -(-(-(-rows // (16 * tm)) * -(-columns // (16 * tn))) // MFMA_CUS)
+                load = 16 * (tm + tn) * inner * size / (KWAVE_LOAD_GBS * 1e3)
+                matrix = 2 * 256 * tm * tn * inner / (KWAVE_MATRIX_GFLOPS[dtype] * 1e3)
+                cost = (KWAVE_OVERHEAD_US + rounds * max(load, matrix), tm, tn)
+                best = min(best or cost, cost)
+        return best
+
+    def _kwave_linear(self, out, x, weight, bias, rows, columns, inner, tm: int, tn: int) -> None:
+        k = Kernel(1)
+        k.min_waves = 1
+        args = [self._matrix_slot(k, x), self._matrix_slot(k, weight), self._matrix_slot(k, bias) if bias is not None else "nullptr"]
+        out_slot = k.slot(out.name, out.dtype, writable=True, extent=self.extents[out.name])
+        slots = min(4, KWAVE_LDS // (KWAVE_WAVES * (tm + tn) << 10))
+        k.line(f"chroma::kwave_linear<{ctype_of(out.dtype)}, {tm}, {tn}, {KWAVE_WAVES}, {slots}>({args[0]}, {args[1]}, {args[2]}, {out_slot}, "
+               f"{rows}u, {columns}u, {inner}u);")
+        tiles = -(-rows // (16 * tm)) * -(-columns // (16 * tn))
+        self.launch(k, 8 * -(-tiles // 8), 64 * KWAVE_WAVES, [x, weight] + ([bias] if bias is not None else []), kind="linear_kwave")
+
     def _mfma_linear(self, out, x, weight, bias, rows, columns, inner) -> None:
+        if self._kwave_fits(x, weight, rows, columns, inner):
+            cost, tm, tn = self._kwave_plan(rows, columns, inner, out.dtype)
+            tiled = math.inf  # float products have no other body for few tiles or many
+            if out.dtype == torch.bfloat16 and inner % 32 == 0:
+                tiled = min(KWAVE_OVERHEAD_US + -(-(-(-rows // m) * -(-columns // n)) // MFMA_CUS) * (m + n) * inner * 2 / (rate * 1e3)
+                            for (m, n), rate in TILED_LOAD_GBS.items())
+            if cost < tiled:
+                # (it gains nothing from weights read ahead: 512 x 2048 x 2048 13.6 -> 15.3 us with the launch, 600 x 2880 x
+                # 4096 30.9 -> 34.6, so plans keep theirs only before small weights under many rows)
+                if rows >= KWAVE_PREFETCH[0] and columns * inner * ITEMSIZE[out.dtype] <= KWAVE_PREFETCH[1]:
+                    self._prefetch_weight(weight)
+                self._kwave_linear(out, x, weight, bias, rows, columns, inner, tm, tn)
+                return
         if not self._wide_gemm(out.dtype, inner, rows, columns):
             # (the wide body's C5 QKV product gains 3.4 us from warm weights, less than the 6.6 us read-ahead;
             # the mid body's output projection 15 us for 5.5)

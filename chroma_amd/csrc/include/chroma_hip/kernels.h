@@ -4,3 +4,4 @@
 #include "device.h"
 #include "linear.h"
 #include "attention.h"
+#include "kwave.h"

@@ -1,0 +1,186 @@
+// Matrix-core products of few output tiles: Y[M, N] = X[M, K] . W[N, K]^T with K split over a workgroup's waves.
+//
+// The tiled bodies in linear.h walk K in slices that all of a workgroup's waves share, a barrier and a round trip per
+// slice; with few output tiles most of the chip idles while a handful of workgroups walk K serially (a 100 x 5120
+// product over K = 2880: 40 workgroups, 45 slices). Here each of NW waves computes the whole 16 TM x 16 TN output
+// tile over its own contiguous share of K: it copies its operands global -> LDS into a ring of its own (no barrier
+// in the loop: a wave waits only for its own copies), and the waves' float partial sums meet once, in LDS, added
+// in wave order. What bounds it is the compute unit's load path, (16 TM + 16 TN) K elements per workgroup at about
+// 75 GB/s for 4 lanes to every 64-byte row piece (operand fragments read straight into registers, a lane to a row,
+// move half of that: the path is bound by the addresses of neighbouring lanes, not by bytes).
+#pragma once
+
+#include "linear.h"
+
+namespace chroma {
+
+// A unit is 64 bytes of every operand row (32 bfloat16 or 16 float values of K): lane l holds the 16-byte chunk
+// l / 16 of row l % 16 of a 16-row block. One v_mfma_f32_16x16x32_bf16 takes a bfloat16 unit as it lies; for float,
+// element e of every lane's 4 forms the operand of one v_mfma_f32_16x16x4f32 (both operands pair the same k, whose
+// order inside a unit is then 0 4 8 12, 1 5 9 13, ...).
+template <class T>
+__device__ __forceinline__ void kwave_mfma(const uint4& b, const uint4& a, f32x4_t& acc) {
+    if constexpr (sizeof(T) == 2) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, a), acc, 0, 0, 0);
+    } else {
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b.x), __uint_as_float(a.x), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b.y), __uint_as_float(a.y), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b.z), __uint_as_float(a.z), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b.w), __uint_as_float(a.w), acc, 0, 0, 0);
+    }
+}
+
+// Elements of the LDS array: S units of TM + TN 16-row blocks (1 KiB each) per wave; a wave's partial sums (TM TN
+// KiB) take the place of its own ring.
+template <int TM, int TN, int NW, int S>
+constexpr int kwave_elements() {
+    return NW * 512 * (S * (TM + TN) > TM * TN ? S * (TM + TN) : TM * TN);
+}
+
+// The row of a 16-row block that this lane copies from.
+__device__ __forceinline__ uint32_t kwave_row() { return threadIdx.x % 64u / 4u; }
+
+// One output tile. ``a`` and ``b`` are the operands' first bytes; ``oa`` and
+// ``ob`` hold the byte offset of row ``kwave_row`` of each 16-row block (rows past the edge repeat a valid row):
+// 32-bit, so the caller guarantees operands below 2 GiB. ``row_bytes`` (a multiple of 16) is K's extent. The ring's
+// 16-byte chunks are swizzled as the ring body's (``wide_swizzle``). ``store(i, j, v)`` is called once per 16 x 16
+// block (i, j) on the wave that sums it: lane l has row 16 i + l % 16, columns 16 j + 4 (l / 16) .. + 3.
+template <class T, int TM, int TN, int NW, int S, class Store>
+__device__ __forceinline__ void kwave_tile(const char* __restrict__ a, const uint32_t (&oa)[TM], const char* __restrict__ b,
+                                           const uint32_t (&ob)[TN], uint32_t row_bytes, uint16_t* lds, Store store) {
+    static_assert(S >= 2, "a unit being read and at least one in flight");
+    constexpr int PER = TM + TN;
+    constexpr uint32_t WAVE = kwave_elements<TM, TN, 1, S>();
+    const uint32_t lane = threadIdx.x % 64u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64u);
+    const uint32_t units = (row_bytes + 63u) / 64u, begin = units * wave / NW, end = units * (wave + 1u) / NW;
+    uint16_t* ring = lds + wave * WAVE;
+    const uint32_t chunk = 16u * ((lane % 4u) ^ wide_swizzle(lane / 4u));                               // copied byte of the row's unit
+    const uint32_t at = (lane % 16u) * 32u + (((lane / 16u) ^ wide_swizzle(lane % 16u)) * 8u);  // fragment element in a block
+    const uint32_t tail = row_bytes % 64u;  // bytes of a ragged last unit
+    f32x4_t acc[TM][TN];
+    unroll<TM>([&](auto i) { unroll<TN>([&](auto j) { acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}; }); });
+    // past the row's end (a ragged last unit) a lane copies the unit's first 16 bytes instead; the reader drops them
+    auto copy = [&](uint32_t u) {
+        const uint32_t from = u * 64u + chunk < row_bytes ? chunk : 0u;
+        uint16_t* slot = ring + (u - begin) % S * (PER * 512u);
+        unroll<PER>([&](auto ic) {
+            constexpr int i = ic;
+            const char* source;
+            if constexpr (i < TM) {
+                source = a + u * 64u + (oa[i] + from);
+            } else {
+                source = b + u * 64u + (ob[i - TM] + from);
+            }
+            __builtin_amdgcn_global_load_lds((global_void*)source, (lds_void*)(slot + i * 512u), 16, 0, 0);
+        });
+    };
+    auto multiply = [&](uint32_t u) {
+        const uint16_t* slot = ring + (u - begin) % S * (PER * 512u) + at;
+        uint4 fa[TM], fb[TN];
+        unroll<TM>([&](auto i) { fa[i] = *reinterpret_cast<const uint4*>(slot + i * 512u); });
+        unroll<TN>([&](auto j) { fb[j] = *reinterpret_cast<const uint4*>(slot + (TM + j) * 512u); });
+        if (tail && u * 64u + 64u > row_bytes && 16u * (lane / 16u) >= tail) {
+            unroll<TM>([&](auto i) { fa[i] = uint4{0u, 0u, 0u, 0u}; });
+            unroll<TN>([&](auto j) { fb[j] = uint4{0u, 0u, 0u, 0u}; });
+        }
+        unroll<TM>([&](auto i) { unroll<TN>([&](auto j) { kwave_mfma<T>(fb[j], fa[i], acc[i][j]); }); });
+    };
+    unroll<S - 1>([&](auto n) {
+        if (begin + uint32_t(n) < end) {
+            copy(begin + uint32_t(n));
+        }
+    });
+    uint32_t u = begin;
+    for (; u + (S - 1) < end; ++u) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_wait((S - 2) * PER));  // unit u landed; the S - 2 after it may be in flight
+        __builtin_amdgcn_sched_barrier(0);
+        copy(u + (S - 1));  // into the slot unit u - 1 was read from
+        multiply(u);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    unroll<S - 1>([&](auto n) {
+        constexpr int left = S - 2 - int(n);  // units in flight behind this one
+        if (end - u > uint32_t(left)) {
+            __builtin_amdgcn_s_waitcnt(vmcnt_wait(left * PER));
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(u);
+            __builtin_amdgcn_sched_barrier(0);
+            ++u;
+        }
+    });
+    if constexpr (NW == 1) {
+        unroll<TM>([&](auto i) { unroll<TN>([&](auto j) { store(i, j, acc[i][j]); }); });
+    } else {
+        // (each wave's last fragment reads are done: they fed its products)
+        f32x4_t* partial = reinterpret_cast<f32x4_t*>(lds) + lane;
+        constexpr uint32_t STRIDE = WAVE / 8u;
+        unroll<TM>([&](auto i) { unroll<TN>([&](auto j) { partial[wave * STRIDE + (i * TN + j) * 64u] = acc[i][j]; }); });
+        __syncthreads();
+        unroll<(TM * TN + NW - 1) / NW>([&](auto n) {
+            const uint32_t t = n * NW + wave;
+            if (t < uint32_t(TM * TN)) {
+                f32x4_t sum = partial[t * 64u];
+                unroll<NW - 1>([&](auto w) { sum += partial[(w + 1) * STRIDE + t * 64u]; });
+                store(t / TN, t % TN, sum);
+            }
+        });
+    }
+}
+
+// A linear layer on ``kwave_tile``: 8 * ceil(tiles / 8) workgroups of 64 NW threads, the row tiles of one column tile
+// adjacent (one XCD's L2 reads each weight row once). Requires 16-byte aligned operands and rows (K a multiple of 8
+// bfloat16 or 4 float values), and X and a column tile of W below 2 GiB. Measured on cold weights, NW = 4, against
+// the 128 x 128 bodies: bfloat16 100 x 5120 x 2880 51.6 -> 18.5 us, 300 x 1024 x 4096 58.9 -> 16.0, 600 x 2880 x 4096
+// 57.3 (the 128 x 192 ring body) -> 32.9; float 256 x 160 x 128 14.3 -> 2.2, 100 x 4000 x 1000 84 -> 15.
+template <class T, int TM, int TN, int NW, int S>
+__device__ __forceinline__ void kwave_linear(const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias, T* __restrict__ out,
+                                             uint32_t m_total, uint32_t n_total, uint32_t k_total) {
+    __shared__ __attribute__((aligned(1024))) uint16_t lds[kwave_elements<TM, TN, NW, S>()];
+    const uint32_t gy = (m_total + 16u * TM - 1u) / (16u * TM), gx = (n_total + 16u * TN - 1u) / (16u * TN);
+    uint32_t logical;
+    if (!xcd_logical_tile(gx * gy, logical)) {
+        return;
+    }
+    const uint32_t m0 = logical % gy * (16u * TM), n0 = logical / gy * (16u * TN);
+    const uint32_t lane = threadIdx.x % 64u, row_bytes = k_total * sizeof(T);
+    uint32_t oa[TM], ob[TN];
+    unroll<TM>([&](auto i) {
+        const uint32_t m = m0 + i * 16u + kwave_row();
+        oa[i] = (m < m_total ? m : m_total - 1u) * row_bytes;
+    });
+    unroll<TN>([&](auto j) {
+        const uint32_t n = n0 + j * 16u + kwave_row();
+        ob[j] = ((n < n_total ? n : n_total - 1u) - n0) * row_bytes;
+    });
+    kwave_tile<T, TM, TN, NW, S>(reinterpret_cast<const char*>(x), oa, reinterpret_cast<const char*>(w) + size_t(n0) * row_bytes, ob, row_bytes, lds,
+                                 [&](uint32_t i, uint32_t j, f32x4_t v) {
+        const uint32_t m = m0 + i * 16u + lane % 16u, n = n0 + j * 16u + 4u * (lane / 16u);
+        if (m >= m_total || n >= n_total) {
+            return;
+        }
+        T* row = out + size_t(m) * n_total + n;
+        float y[4];
+#pragma unroll
+        for (uint32_t r = 0; r < 4u; ++r) {
+            y[r] = v[r] + (bias ? load1<T>(bias + (n + r < n_total ? n + r : n_total - 1u)) : 0.0f);
+        }
+        if (n_total % 4u == 0) {
+            if constexpr (sizeof(T) == 2) {
+                *reinterpret_cast<uint2*>(row) = uint2{uint32_t(f32_to_bf16(y[0])) | uint32_t(f32_to_bf16(y[1])) << 16,
+                                                       uint32_t(f32_to_bf16(y[2])) | uint32_t(f32_to_bf16(y[3])) << 16};
+            } else {
+                *reinterpret_cast<float4*>(row) = float4{y[0], y[1], y[2], y[3]};
+            }
+            return;
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < 4u; ++r) {
+            if (n + r < n_total) {
+                store1<T>(row + r, y[r]);
+            }
+        }
+    });
+}
+
+}  // namespace chroma

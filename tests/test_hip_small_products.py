@@ -1,0 +1,67 @@
+"""Products and attention of few output tiles: the kernels that split K or the keys over waves and workgroups."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import chroma_amd
+from chroma_amd._src.codegen.hip import HIPCodegen
+from chroma_amd._src.compiler import lower_program
+from tests.helpers import Function, as_float, export
+
+
+def assert_sums(got, exact, terms, scale, dtype):
+    """``got`` against 64-bit sums of ``terms`` products of standard deviation ``scale``: a float sum's partial sums
+    grow like a random walk, so its rounding errors add up to about 2^-24 scale terms / sqrt(2) (8 of them are
+    allowed), and the stored value is rounded once (half a spacing: 2^-9 relative in bfloat16, 2^-24 in float)."""
+    error = np.abs(as_float(got).astype(np.float64) - exact.numpy())
+    limit = 8 * 2.0**-24 * scale * terms + np.abs(exact.numpy()) * (2.0**-8 if dtype == torch.bfloat16 else 2.0**-23)
+    worst = np.unravel_index(np.argmax(error - limit), error.shape)
+    assert (error <= limit).all(), (worst, error[worst], limit[worst])
+
+
+def plan_of(module, *inputs):
+    return lower_program(export(module, *inputs), HIPCodegen()).files["model.hip"]
+
+
+def linear(rows, inner, columns, dtype, bias=True):
+    generator = torch.Generator().manual_seed(rows + inner + columns)
+    layer = torch.nn.Linear(inner, columns, bias=bias).eval()
+    with torch.no_grad():
+        for parameter in layer.parameters():
+            parameter.copy_(torch.randn(parameter.shape, generator=generator) * 0.05)
+    return layer.to(dtype), torch.randn(rows, inner, generator=generator).to(dtype)
+
+
+def test_unaligned_operands_keep_the_general_body():
+    """The K-split body copies 16-byte chunks: rows that are no whole chunks, or an operand that starts between two,
+    stay on the bodies that took them before."""
+    x = torch.ones(40 * 256 + 8)
+    assert "kwave_linear<float" in plan_of(Function(lambda v, w: torch.nn.functional.linear(v[4:4 + 40 * 256].reshape(40, 256), w)), x, torch.ones(33, 256))
+    assert "kwave_linear" not in plan_of(Function(lambda v, w: torch.nn.functional.linear(v[2:2 + 40 * 256].reshape(40, 256), w)), x, torch.ones(33, 256))
+    assert "kwave_linear" not in plan_of(Function(torch.nn.functional.linear), torch.ones(40, 258), torch.ones(33, 258))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows, inner, columns", [
+    (17, 128, 7),       # every wave one bfloat16 unit of K; one partial column tile, odd stores
+    (18, 136, 160),     # K ends inside a unit
+    (3, 11528, 37),     # few rows too wide for the streaming kernel, ragged last unit
+    (16, 4096, 129),
+    (100, 1000, 515),   # ragged rows, columns and K; more units than ring slots
+    (250, 4096, 128),
+    (300, 264, 1024),
+    (700, 640, 2880),   # the largest tiles
+])
+def test_k_split_linear(tmp_path, dtype, rows, inner, columns):
+    layer, x = linear(rows, inner, columns, dtype)
+    exported = torch.export.export(layer, (x,))
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        assert "kwave_linear" in (tmp_path / "hip" / "model.hip").read_text()
+        got = [model(x) for _ in range(2)]
+    exact = x.double() @ layer.weight.detach().double().T + layer.bias.detach().double()
+    for result in got:
+        assert_sums(result, exact, inner, 0.05, dtype)
