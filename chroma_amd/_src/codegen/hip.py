@@ -2270,6 +2270,9 @@ class HIPCodegen(Codegen):
         keys = past + k_new.shape[0]
         out = self.allocate(tuple(meta.shape), meta.dtype)
         bf16 = meta.dtype == torch.bfloat16
+        if self.blas and bf16 and dim in (32, 64, 128) and self._flash_rows(tokens, kv_heads, group, keys):
+            if self._flash_attention(out, q, k_past, k_new, v_past, v_new, mask, sinks, scale):
+                return out
         if self.blas and bf16 and dim % 32 == 0 and dim <= 128 and tokens >= MATRIX_ATTENTION_TOKENS:
             if self._matrix_attention(out, q, k_past, k_new, v_past, v_new, mask, sinks, scale):
                 return out
@@ -2311,6 +2314,16 @@ class HIPCodegen(Codegen):
             self.launch(k, (tokens, kv_heads, 1), 256, [partial], kind="attention_combine")
         self.fused_attentions += 1
         return out
+
+    @staticmethod
+    def _flash_rows(tokens: int, kv_heads: int, group: int, keys: int) -> bool:
+        """Whether an attention of these extents goes to ``attention_flash_bf16``: below MATRIX_ATTENTION_TOKENS queries
+        every one but a decode step over a long cache (one query over more than 4 decode splits of keys has kernels of
+        its own); from there on those whose 16-query tiles would leave compute units idle and whose keys are enough
+        to split."""
+        if tokens < MATRIX_ATTENTION_TOKENS:
+            return tokens > 1 or keys <= 4 * DECODE_SPLIT_KEYS
+        return keys > 4 * DECODE_SPLIT_KEYS and kv_heads * -(-tokens // 16) < MFMA_CUS
 
     def _waves_attention(self, out, q, k_past, k_new, v_past, v_new, mask, sinks, scale, epilogue=None) -> Kernel:
         """The one-wave-per-query-head attention kernel. ``epilogue`` = (weight, bias, linear output, lanes,
@@ -2594,9 +2607,9 @@ class HIPCodegen(Codegen):
         broadcast = [0] * pad + [0 if size == 1 else stride for size, stride in zip(value.shape, strides)]
         return stored, broadcast, stored.view.offset if stored.view.base is not None else 0
 
-    def _matrix_attention(self, out, q, k_past, k_new, v_past, v_new, mask, sinks, scale) -> bool:
-        """The long-prefill attention on the matrix cores (``attention_mfma_bf16``); False (nothing
-        emitted) when an operand's layout does not allow 16-byte rows."""
+    def _attention_plan(self, q, k_past, k_new, v_past, v_new, mask, sinks) -> Optional[dict]:
+        """The operands of a matrix-core attention read in place: {name: (stored value, element strides, offset)},
+        expressions stored; None (nothing stored) when an operand's layout does not allow 16-byte rows."""
         tokens, kv_heads, group, dim = q.shape
         past = k_past.shape[0] if k_past is not None else 0
         keys = past + k_new.shape[0]
@@ -2613,14 +2626,18 @@ class HIPCodegen(Codegen):
             strides = [0] * pad + [0 if size == 1 else stride for size, stride in zip(value.shape, strides)]
             offset = stored.view.offset if stored is not None and stored.view.base is not None else 0
             if name in ("q", "k_new", "v_new", "k_past", "v_past") and (strides[-1] != 1 or any(x % 8 for x in strides[:-1]) or offset % 8):
-                return False
+                return None
             if (name == "mask" and strides[3] != 1) or (name == "sinks" and strides[2] != 0):
-                return False
+                return None
         plan = {name: self._operand(value, shape) for name, (value, shape) in operands.items()}
         plan.setdefault("k_past", None)
         plan.setdefault("v_past", None)
+        return plan
+
+    def _attention_operands(self, k: Kernel, out: Value, plan: dict, q: Value, past: int, keys: int, scale: float) -> None:
+        """``chroma::AttentionOperands a`` of ``plan``."""
+        tokens, kv_heads, group, _ = q.shape
         q_strides, mask_strides, sink_strides = plan["q"][1], plan["mask"][1], plan["sinks"][1]
-        k = Kernel(1)
         slot = k.slot(out.name, out.dtype, writable=True, extent=self.extents[out.name])
 
         def pointer(name: str) -> str:
@@ -2644,14 +2661,71 @@ class HIPCodegen(Codegen):
         k.line(f"a.sinks = {pointer('sinks')}; a.sh = {sink_strides[0]}u; a.sg = {sink_strides[1]}u;")
         k.line(f"a.out = {slot}; a.tokens = {tokens}u; a.past = {past}u; a.keys = {keys}u; a.kv_heads = {kv_heads}u; a.group = {group}u;")
         k.line(f"a.scale = {float_literal(scale)};")
+
+    @staticmethod
+    def _power_of_two(scale: float) -> bool:
+        """A power-of-two scale <= 1 makes the scaled score a bfloat16 value: its rounding is left out."""
+        mantissa, exponent = math.frexp(scale)
+        return mantissa == 0.5 and -64 <= exponent <= 1
+
+    def _flash_attention(self, out, q, k_past, k_new, v_past, v_new, mask, sinks, scale) -> bool:
+        """bfloat16 attention of few query rows on the matrix cores with the keys split over waves and workgroups
+        (``attention_flash_bf16``); False (nothing emitted) when an operand's layout or the mask does not allow it."""
+        tokens, kv_heads, group, dim = q.shape
+        past = k_past.shape[0] if k_past is not None else 0
+        keys = past + k_new.shape[0]
+        # one mask for every head (the check of ``_attention_plan`` on its broadcast strides, before anything is stored)
+        if any(size != 1 for size in mask.shape[:-2]) or len(mask.shape) < 2:
+            return False
+        plan = self._attention_plan(q, k_past, k_new, v_past, v_new, mask, sinks)
+        if plan is None:
+            return False
+        tiles = 2 if tokens * group > 16 else 1  # 16-row tiles per wave: two share each K and V fragment
+        groups = -(-tokens * group // (16 * tiles))
+        blocks = -(-keys // 64)
+        # as many splits as bring the launch to one workgroup of 4 waves per compute unit, each wave a block at least
+        splits = max(1, min(-(-blocks // 4), MFMA_CUS // (kv_heads * groups)))
+        operands = [entry[0] for entry in plan.values() if entry is not None]
+        partial = self.allocate((kv_heads * groups * splits * 16 * tiles * (dim + 2),), torch.float32) if splits > 1 else None
+        k = Kernel(1)
+        k.min_waves = 1
+        self._attention_operands(k, out, plan, q, past, keys, scale)
+        scratch = k.slot(partial.name, torch.float32, writable=True, extent=self.extents[partial.name]) if partial is not None else "nullptr"
+        quads = not (plan["mask"][1][2] % 4 or plan["mask"][2] % 4 or keys % 4)
+        k.line(f"chroma::attention_flash_bf16<{dim}, {group}, {tiles}, {str(self._power_of_two(scale)).lower()}, {str(quads).lower()}>"
+               f"(a, {splits}u, {scratch});")
+        self.launch(k, (kv_heads, groups, splits), 256, operands, kind="attention_flash")
+        if partial is not None:
+            k = Kernel(1)
+            value, strides, offset = plan["sinks"]
+            base = k.slot(value.root.name, value.root.dtype, extent=self.extents[value.root.name])
+            slot = k.slot(out.name, out.dtype, writable=True, extent=self.extents[out.name])
+            scratch = k.slot(partial.name, torch.float32, extent=self.extents[partial.name])
+            k.line(f"chroma::attention_flash_combine<{dim}, {group}, {tiles}>({scratch}, {base} + {offset}u, {strides[0]}u, {strides[1]}u, {slot}, {tokens}u, {splits}u);")
+            self.launch(k, (kv_heads, groups, 1), 256, [partial, value], kind="attention_flash_combine")
+        self.fused_attentions += 1
+        if tokens >= MATRIX_ATTENTION_TOKENS:
+            self.mfma_matmuls += 1
+        return True
+
+    def _matrix_attention(self, out, q, k_past, k_new, v_past, v_new, mask, sinks, scale) -> bool:
+        """The long-prefill attention on the matrix cores (``attention_mfma_bf16``); False (nothing
+        emitted) when an operand's layout does not allow 16-byte rows."""
+        tokens, kv_heads, group, dim = q.shape
+        past = k_past.shape[0] if k_past is not None else 0
+        keys = past + k_new.shape[0]
+        plan = self._attention_plan(q, k_past, k_new, v_past, v_new, mask, sinks)
+        if plan is None:
+            return False
+        mask_strides = plan["mask"][1]
+        k = Kernel(1)
+        self._attention_operands(k, out, plan, q, past, keys, scale)
         shared_mask = mask_strides[0] == mask_strides[1] == 0
         if shared_mask and group <= 8:
             # one workgroup per (16-query tile, KV head), one wave per query head: K/V/mask tiles staged once
             live = self._live_blocks(plan["mask"], tokens, keys, tile=(16, 64))
             k.line(f"a.live_blocks = reinterpret_cast<const uint8_t*>({k.slot(live.name, torch.int64, extent=self.extents[live.name])});")
-            # a power-of-two scale <= 1 makes the scaled score a bfloat16 value: its rounding is left out
-            mantissa, exponent = math.frexp(scale)
-            pow2 = mantissa == 0.5 and -64 <= exponent <= 1
+            pow2 = self._power_of_two(scale)
             # (head dimensions above 64 would need more registers than three workgroups per CU leave)
             per_wave = ATTENTION_HEADS_PER_WAVE if group % ATTENTION_HEADS_PER_WAVE == 0 and dim <= 64 else 1
             k.min_waves = ATTENTION_HEADS_MIN_BLOCKS if per_wave > 1 else 0

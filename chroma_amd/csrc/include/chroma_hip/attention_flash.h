@@ -1,0 +1,374 @@
+// bfloat16 grouped-query attention with sinks for few query rows: the chain of attention.h on the matrix cores, one
+// pass over the keys, each wave on key blocks of its own.
+//
+// The group-shared kernel (``attention_heads_mfma_bf16``) gives a workgroup 16 queries and every key; with few queries
+// the chip idles (100 queries x 8 heads: 56 workgroups), and below 16 queries most of a tile is padding. Here a tile is
+// 16 (query, head of the group) rows, so one query of 8 heads fills half of one and 36 queries 18, and the keys are
+// split over the 4 waves of a workgroup and over ``splits`` workgroups. A wave copies its 64-key block of K and of V
+// global -> LDS into buffers of its own (no barrier in the loop), reads V^T fragments with the transposing LDS read,
+// and keeps (max, sum, p . v) of its keys; the waves of a workgroup meet in LDS, workgroups through ``partial`` (added
+// by ``attention_flash_combine``). What bounds it is latency: a block's copies, one round trip, behind the block before.
+// Measured on 8 KV heads of 8 heads of 64 (kernel time, before -> with the combining launch): 3 queries over 137 keys
+// 134 -> 5 us, 36 over 4072 (128-key windows) 848 -> 13, 100 over 1100 23 + 5 (live tiles) -> 9; a whole layer's call of
+// 400 queries over 2401 keys 208 -> 150 us (with its products), 480 over 4481 307 -> 220.
+//
+// Rounding: the scores, scaled scores and masked scores are rounded as attention.h says; a probability is rounded to
+// bfloat16 as exp(s - m), m a running maximum of the row, before it meets V, and the row is divided by the float sum at
+// the end (the same relative rounding of each probability as when it is divided first).
+#pragma once
+
+#include "attention.h"
+
+namespace chroma {
+
+constexpr uint32_t kFlashWaves = 4, kFlashKeys = 64;
+// A wave's maximum is only raised (its sums rescaled) once a score exceeds it by more than this: probabilities then
+// stay below e^8, far inside float and bfloat16 range.
+constexpr float kFlashHeadroom = 8.0f;
+
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
+
+// Floats of one (KV head, row group, split): per row the maximum and the sum, then the D sums of p . v.
+template <int D, int RT> constexpr uint32_t flash_partial_floats() { return 16u * RT * (D + 2u); }
+
+// The result of a row from its (max, sum, p . v) parts: weights exp(max_i - M) with M the largest of them and the sink.
+// A row whose scores and sink are all -inf divides 0 by 0, as the reference does.
+struct FlashMerge {
+    float top, total;
+    __device__ __forceinline__ float weight(float peak) const { return peak == -__builtin_inff() ? 0.0f : fast_exp(peak - top); }
+};
+
+// MASK4: the mask's rows, first element and key count are multiples of 4 elements, so its entries are read 4 at a time.
+template <int D, int G, int RT, bool POW2, bool MASK4>
+__device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a, uint32_t splits, float* __restrict__ partial) {
+    static_assert(D % 32 == 0 && D <= 128 && G >= 1, "head dimension and group");
+    constexpr uint32_t WAVE = 2u * kFlashKeys * D;  // LDS elements per wave: a K block and a V block
+    constexpr uint32_t ROWS = 16u * RT, OPAD = D + 4u;
+    static_assert(ROWS * (OPAD + 2u) * 2u <= WAVE, "a wave's sums fit its buffers");
+    constexpr int COPIES = kFlashKeys * D / 512;   // 1 KB copies per block and operand
+    constexpr uint32_t PER_ROW = D / 8u;           // 16-byte chunks of a key's row
+    constexpr uint32_t SWZ = PER_ROW % 8u == 0 ? 7u : 3u;  // chunk c of row r lies at c ^ ((r / 2) & SWZ)
+    constexpr float kLog2e = 1.44269504088896341f;
+    __shared__ __attribute__((aligned(1024))) uint16_t lds[kFlashWaves * WAVE];
+    const uint32_t lane = threadIdx.x % 64u, quad = lane / 16u, col = lane % 16u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64u);
+    const uint32_t kv = blockIdx.x, row0 = blockIdx.y * ROWS, split = blockIdx.z;
+    const uint32_t total_rows = a.tokens * G;
+    const float neg_inf = -__builtin_inff();
+    uint16_t* ks = lds + wave * WAVE;
+    uint16_t* vs = ks + kFlashKeys * D;
+
+    uint32_t query[RT];
+    bf16x8_t qf[RT][D / 32];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const uint32_t row = row0 + rt * 16u + col < total_rows ? row0 + rt * 16u + col : total_rows - 1u;
+        query[rt] = row / G;
+#pragma unroll
+        for (int c = 0; c < D / 32; ++c) {
+            qf[rt][c] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(a.q + size_t(query[rt]) * a.qt + kv * a.qh + (row % G) * a.qg + c * 32u + quad * 8u));
+        }
+    }
+
+    // This wave's key blocks: split * 4 + wave, then every 4 * splits. With more than one, those that a mask entry of
+    // this group's queries leaves alive are found first (a bit each; past 64 they all count as alive).
+    const uint32_t blocks = (a.keys + kFlashKeys - 1u) / kFlashKeys, stride = kFlashWaves * splits, first = split * kFlashWaves + wave;
+    const uint32_t mine = first < blocks ? (blocks - first + stride - 1u) / stride : 0u;
+    unsigned long long alive = ~0ull;
+    if (mine > 1u) {
+        constexpr int TQ = (ROWS + G - 1) / G + 1;  // queries a group's rows can touch
+        const uint32_t q_first = row0 / G, q_last = (row0 + ROWS < total_rows ? row0 + ROWS - 1u : total_rows - 1u) / G;
+        alive = 0ull;
+        for (uint32_t n0 = 0; n0 < (mine < 64u ? mine : 64u); n0 += 4u) {
+            uint16_t bits[4][TQ];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t j = (first + (n0 + i) * stride) * kFlashKeys + lane;
+#pragma unroll
+                for (int t = 0; t < TQ; ++t) {
+                    const uint32_t q = q_first + t < q_last ? q_first + t : q_last;
+                    bits[i][t] = a.mask[size_t(q) * a.mt + (j < a.keys ? j : a.keys - 1u)];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                bool any = false;
+#pragma unroll
+                for (int t = 0; t < TQ; ++t) {
+                    any |= bits[i][t] != 0xff80u;
+                }
+                any = any && n0 + i < mine && (first + (n0 + i) * stride) * kFlashKeys + lane < a.keys;
+                if (__ballot(any) != 0ull) {
+                    alive |= 1ull << (n0 + i);
+                }
+            }
+        }
+    }
+    auto next_of = [&](uint32_t n) {
+        while (n < mine && n < 64u && !((alive >> n) & 1ull)) {
+            ++n;
+        }
+        return n;
+    };
+
+    // Copies: lane l moves position l % PER_ROW of row l / PER_ROW of each 1 KB piece. Keys past the end repeat the last.
+    auto copy = [&](uint16_t* to, const uint16_t* past, uint32_t pj, uint32_t ph, const uint16_t* fresh, uint32_t nj, uint32_t nh, uint32_t block) {
+#pragma unroll
+        for (int i = 0; i < COPIES; ++i) {
+            const uint32_t r = i * (64u / PER_ROW) + lane / PER_ROW, chunk = (lane % PER_ROW) ^ ((r / 2u) & SWZ);
+            const uint32_t j = block * kFlashKeys + r < a.keys ? block * kFlashKeys + r : a.keys - 1u;
+            const bool old = j < a.past;
+            const uint16_t* row = old ? past + (size_t(j) * pj + kv * ph) : fresh + (size_t(j - a.past) * nj + kv * nh);
+            __builtin_amdgcn_global_load_lds((global_void*)(row + chunk * 8u), (lds_void*)(to + i * 512u), 16, 0, 0);
+        }
+    };
+    auto copy_k = [&](uint32_t block) { copy(ks, a.k_past, a.kpj, a.kph, a.k_new, a.knj, a.knh, block); };
+    auto copy_v = [&](uint32_t block) { copy(vs, a.v_past, a.vpj, a.vph, a.v_new, a.vnj, a.vnh, block); };
+
+    float peak[RT], total[RT];
+    f32x4_t o[RT][D / 16];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        peak[rt] = neg_inf;
+        total[rt] = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) {
+            o[rt][dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    uint32_t n = next_of(0);
+    if (n < mine) {
+        copy_k(first + n * stride);
+        copy_v(first + n * stride);
+    }
+    while (n < mine) {
+        const uint32_t block = first + n * stride, next = next_of(n + 1u);
+        // mask entries of this lane: keys 16 t + 4 quad .. + 3 of the block, its query
+        // (every load unconditional, clamped: a guarded load would end its branch with a wait)
+        uint2 m[RT][4];
+        uint16_t element[RT][4][4];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const uint32_t j = block * kFlashKeys + t * 16u + quad * 4u;
+                const uint16_t* row = a.mask + size_t(query[rt]) * a.mt;
+                if constexpr (MASK4) {
+                    m[rt][t] = *reinterpret_cast<const uint2*>(row + (j < a.keys ? j : a.keys - 4u));
+                } else {
+#pragma unroll
+                    for (uint32_t r = 0; r < 4u; ++r) {
+                        element[rt][t][r] = row[j + r < a.keys ? j + r : a.keys - 1u];
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));  // K, V and the mask of this block
+        __builtin_amdgcn_sched_barrier(0);
+        // scores of keys 16 t + 4 quad + r for this lane's row, in u units: s = u * cs (attention_heads_mfma_bf16)
+        float u[RT][4][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x4_t s[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                s[rt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                const uint32_t j = block * kFlashKeys + t * 16u + quad * 4u;
+                if constexpr (!MASK4) {
+                    uint32_t e[4];
+#pragma unroll
+                    for (uint32_t r = 0; r < 4u; ++r) {
+                        e[r] = j + r < a.keys ? uint32_t(element[rt][t][r]) : 0xff80u;
+                    }
+                    m[rt][t] = uint2{e[0] | e[1] << 16, e[2] | e[3] << 16};
+                } else if (j >= a.keys) {
+                    m[rt][t] = uint2{0xff80ff80u, 0xff80ff80u};
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < D / 32; ++c) {
+                const uint32_t r = t * 16u + col;
+                const bf16x8_t kf = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(ks + r * D + ((c * 4u + quad) ^ ((r / 2u) & SWZ)) * 8u));
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    s[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][c], s[rt], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    float x = s[rt][r], y = s[rt][r + 1];
+                    round_bf16_pair(x, y);
+                    x *= a.scale;
+                    y *= a.scale;
+                    if constexpr (!POW2) {
+                        round_bf16_pair(x, y);
+                    }
+                    const uint32_t w = r == 0 ? m[rt][t].x : m[rt][t].y;
+                    x += __uint_as_float(w << 16);
+                    y += __uint_as_float(w & 0xffff0000u);
+                    round_bf16_pair(x, y);
+                    u[rt][t][r] = x;
+                    u[rt][t][r + 1] = y;
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        bf16x8_t pf[RT][2];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            float top = neg_inf;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                top = __builtin_fmaxf(top, __builtin_fmaxf(__builtin_fmaxf(u[rt][t][0], u[rt][t][1]), __builtin_fmaxf(u[rt][t][2], u[rt][t][3])));
+            }
+            if (__ballot(top > peak[rt] + kFlashHeadroom || (peak[rt] == neg_inf && top != neg_inf)) != 0ull) {
+                top = __builtin_fmaxf(top, __shfl_xor(top, 16, kWave));
+                top = __builtin_fmaxf(top, __shfl_xor(top, 32, kWave));
+                top = __builtin_fmaxf(top, peak[rt]);
+                const float shrink = peak[rt] == neg_inf ? 0.0f : fast_exp(peak[rt] - top);
+                total[rt] *= shrink;
+#pragma unroll
+                for (int dt = 0; dt < D / 16; ++dt) {
+                    o[rt][dt] *= shrink;
+                }
+                peak[rt] = top;
+            }
+            const float shift = peak[rt] == neg_inf ? 0.0f : -peak[rt] * kLog2e;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                float e[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    e[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(u[rt][t][r], kLog2e, shift));
+                    total[rt] += e[r];
+                }
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    const bf16x2_t pair = __builtin_convertvector(f32x2_t{e[r], e[r + 1]}, bf16x2_t);
+                    pf[rt][t / 2][t % 2 * 4 + r] = pair[0];
+                    pf[rt][t / 2][t % 2 * 4 + r + 1] = pair[1];
+                }
+            }
+        }
+        // slots 0-3 and 4-7 of lane (d, quad) hold keys 32 h + 4 quad + r and 32 h + 16 + 4 quad + r: one transposing
+        // read each (lane 4 r + c of a quad gives the address of key r's columns 4 c .. + 3 and receives column
+        // 4 r + c of the four keys)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) {
+                s16x4_t half[2];
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    const uint32_t r = h * 32u + x * 16u + quad * 4u + col / 4u;
+                    const uint32_t chunk = (dt * 2u + (col % 4u) / 2u) ^ ((r / 2u) & SWZ);
+                    half[x] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vs + r * D + chunk * 8u + (col % 2u) * 4u));
+                }
+                const uint2 lo = __builtin_bit_cast(uint2, half[0]), hi = __builtin_bit_cast(uint2, half[1]);
+                const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, uint4{lo.x, lo.y, hi.x, hi.y});
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[rt][h], o[rt][dt], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // Both buffers have been read. (Copies issued earlier would be waited for by the reads above: the compiler
+        // cannot tell the buffers apart. The other waves of the compute unit cover the round trip.)
+        if (next < mine) {
+            copy_k(first + next * stride);
+            copy_v(first + next * stride);
+        }
+        n = next;
+    }
+
+    // The waves' parts: rows of (D + 4) floats in each wave's own buffers, then [row][max, sum].
+    float* mine_o = reinterpret_cast<float*>(lds + wave * WAVE);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        total[rt] += __shfl_xor(total[rt], 16, kWave);
+        total[rt] += __shfl_xor(total[rt], 32, kWave);
+        const uint32_t r = rt * 16u + col;
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) {
+            *reinterpret_cast<f32x4_t*>(mine_o + r * OPAD + dt * 16u + quad * 4u) = o[rt][dt];
+        }
+        if (quad == 0) {
+            mine_o[ROWS * OPAD + 2u * r] = peak[rt];
+            mine_o[ROWS * OPAD + 2u * r + 1u] = total[rt];
+        }
+    }
+    __syncthreads();
+    const float* parts = reinterpret_cast<const float*>(lds);
+    constexpr uint32_t PART = WAVE / 2u;  // floats of a wave's buffers
+    for (uint32_t i = threadIdx.x; i < ROWS * (D / 4u); i += 64u * kFlashWaves) {
+        const uint32_t r = i / (D / 4u), d = i % (D / 4u) * 4u, row = row0 + r;
+        if (row >= total_rows) {
+            continue;
+        }
+        FlashMerge merge{splits == 1u ? bf16_to_f32(a.sinks[kv * a.sh + (row % G) * a.sg]) : neg_inf, 0.0f};
+        const float sink = merge.top;
+#pragma unroll
+        for (uint32_t w = 0; w < kFlashWaves; ++w) {
+            merge.top = __builtin_fmaxf(merge.top, parts[w * PART + ROWS * OPAD + 2u * r]);
+        }
+        f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (uint32_t w = 0; w < kFlashWaves; ++w) {
+            const float scale = merge.weight(parts[w * PART + ROWS * OPAD + 2u * r]);
+            merge.total += scale * parts[w * PART + ROWS * OPAD + 2u * r + 1u];
+            sum += scale * *reinterpret_cast<const f32x4_t*>(parts + w * PART + r * OPAD + d);
+        }
+        if (splits == 1u) {
+            merge.total += merge.weight(sink);
+            sum *= 1.0f / merge.total;
+            uint16_t* to = a.out + ((size_t(row / G) * a.kv_heads + kv) * G + row % G) * D + d;
+            *reinterpret_cast<uint2*>(to) = uint2{uint32_t(f32_to_bf16(sum[0])) | uint32_t(f32_to_bf16(sum[1])) << 16,
+                                                  uint32_t(f32_to_bf16(sum[2])) | uint32_t(f32_to_bf16(sum[3])) << 16};
+        } else {
+            float* to = partial + size_t((kv * gridDim.y + blockIdx.y) * splits + split) * flash_partial_floats<D, RT>();
+            *reinterpret_cast<f32x4_t*>(to + 2u * ROWS + r * D + d) = sum;
+            if (d == 0) {
+                to[2u * r] = merge.top;
+                to[2u * r + 1u] = merge.total;
+            }
+        }
+    }
+}
+
+// The splits of every row, in order, and the sink (grid: KV heads x row groups, 256 threads).
+template <int D, int G, int RT>
+__device__ __forceinline__ void attention_flash_combine(const float* __restrict__ partial, const uint16_t* __restrict__ sinks, uint32_t sh,
+                                                        uint32_t sg, uint16_t* __restrict__ out, uint32_t tokens, uint32_t splits) {
+    constexpr uint32_t ROWS = 16u * RT, PART = flash_partial_floats<D, RT>();
+    const uint32_t kv = blockIdx.x, row0 = blockIdx.y * ROWS;
+    const float* parts = partial + size_t(kv * gridDim.y + blockIdx.y) * splits * PART;
+    for (uint32_t i = threadIdx.x; i < ROWS * (D / 4u); i += 256u) {
+        const uint32_t r = i / (D / 4u), d = i % (D / 4u) * 4u, row = row0 + r;
+        if (row >= tokens * G) {
+            continue;
+        }
+        const float sink = bf16_to_f32(sinks[kv * sh + (row % G) * sg]);
+        FlashMerge merge{sink, 0.0f};
+        for (uint32_t s = 0; s < splits; ++s) {
+            merge.top = __builtin_fmaxf(merge.top, parts[s * PART + 2u * r]);
+        }
+        f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t s = 0; s < splits; ++s) {
+            const float scale = merge.weight(parts[s * PART + 2u * r]);
+            merge.total += scale * parts[s * PART + 2u * r + 1u];
+            sum += scale * *reinterpret_cast<const f32x4_t*>(parts + s * PART + 2u * ROWS + r * D + d);
+        }
+        merge.total += merge.weight(sink);
+        sum *= 1.0f / merge.total;
+        uint16_t* to = out + ((size_t(row / G) * gridDim.x + kv) * G + row % G) * D + d;
+        *reinterpret_cast<uint2*>(to) = uint2{uint32_t(f32_to_bf16(sum[0])) | uint32_t(f32_to_bf16(sum[1])) << 16,
+                                              uint32_t(f32_to_bf16(sum[2])) | uint32_t(f32_to_bf16(sum[3])) << 16};
+    }
+}
+
+}  // namespace chroma

@@ -4,4 +4,5 @@
 #include "device.h"
 #include "linear.h"
 #include "attention.h"
+#include "attention_flash.h"
 #include "kwave.h"

@@ -65,3 +65,52 @@ def test_k_split_linear(tmp_path, dtype, rows, inner, columns):
     exact = x.double() @ layer.weight.detach().double().T + layer.bias.detach().double()
     for result in got:
         assert_sums(result, exact, inner, 0.05, dtype)
+
+
+def attention_inputs(tokens, past, kv_heads, group, dim, window):
+    """Operands of a cached attention with sinks: causal (or windowed) over a cache of ``past`` rows, one query row
+    wholly masked, an additive bias on a band of keys."""
+    generator = torch.Generator().manual_seed(tokens * 31 + past + dim)
+
+    def rand(*shape, scale=1.0):
+        return (torch.randn(*shape, generator=generator) * scale).to(torch.bfloat16)
+
+    keys = past + tokens
+    mask = torch.zeros(tokens, keys)
+    mask[:, keys // 3 : keys // 3 + 30] = torch.randn(tokens, 30, generator=generator)[:, : keys - keys // 3] * 0.5
+    for t in range(tokens):
+        mask[t, past + t + 1 :] = -torch.inf
+        if window is not None:
+            mask[t, : max(0, past + t - window)] = -torch.inf
+    if tokens > 2:
+        mask[1, :] = -torch.inf
+    return (rand(tokens, kv_heads, group, dim), rand(past, kv_heads, dim), rand(tokens, kv_heads, dim), rand(past, kv_heads, dim),
+            rand(tokens, kv_heads, dim), mask.to(torch.bfloat16), rand(kv_heads * group, scale=2.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens, past, kv_heads, group, dim, window", [
+    (1, 99, 8, 8, 64, None),     # one query, keys a multiple of 4 in a partial block
+    (3, 131, 2, 4, 32, 40),      # 12 of 16 rows; heads of 32
+    (2, 701, 8, 8, 64, 128),     # odd key count, whole key blocks masked, no split
+    (16, 1000, 1, 3, 128, None), # an odd group: rows of one query in two tiles; one KV head, keys split
+    (36, 4036, 8, 8, 64, 128),   # many dead blocks per wave
+    (63, 17, 2, 8, 64, None),
+    (100, 1000, 8, 8, 64, 128),
+    (70, 5000, 1, 8, 64, None),  # several blocks per wave and split
+])
+def test_few_query_attention(tmp_path, tokens, past, kv_heads, group, dim, window):
+    """Attention of few query rows with the keys split over waves and workgroups, against the oracle's unfused chain at
+    its bfloat16 bar, twice."""
+    from oracle import compile_cpu
+    from tests.helpers import assert_close, numpy_of
+    from tests.test_hip_runtime import SinkAttention
+
+    inputs = attention_inputs(tokens, past, kv_heads, group, dim, window)
+    exported = torch.export.export(SinkAttention(), inputs)
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        assert "attention_flash_bf16" in (tmp_path / "hip" / "model.hip").read_text()
+        got = [model(*inputs) for _ in range(2)]
+    want = compile_cpu(exported, tmp_path / "cpu")(*[numpy_of(v) for v in inputs])
+    for result in got:
+        assert_close(result, want, rtol=2e-2, atol=1e-2)
