@@ -114,6 +114,12 @@ TILED_LOAD_GBS = {(256, 192): 36.0, (128, 192): 44.0}
 # rounds of the chip's 256, now with longer tiles among them), on 192 x 4 waves with 160 236 us, but 276 us
 # against 241 us on the skewed routing the seeded C5 model produces (expert counts 0-1842 at layer 19).
 RING_EXPERT_TILES = ((384, 8, 160), (320, 4, 128))
+# With up to FEW_EXPERT_SLOTS slots an expert (mostly one row tile each, a stream over the weights) a product that would take
+# the 320-channel tile takes this one where its channels allow: 2880 channels of 32 experts are then 480 tiles, two nearly
+# full rounds of the chip, instead of 288, one and an eighth (GPT-OSS-20B's layer of 100 tokens 350 -> 324 us, of 400
+# 414 -> 394; at 800 tokens, 100 slots an expert, 499 and 498; 240-, 480- and 160-channel tiles are slower at 100).
+FEW_EXPERT_SLOTS = 64
+FEW_SLOT_TILE = (192, 4, 128)
 # A gated activation between two expert products is computed in the first product's epilogue (no map
 # launch; the first product is not stored when nothing else reads it). False keeps the separate launch.
 ACTIVATION_EPILOGUES = True
@@ -2270,7 +2276,7 @@ class HIPCodegen(Codegen):
         keys = past + k_new.shape[0]
         out = self.allocate(tuple(meta.shape), meta.dtype)
         bf16 = meta.dtype == torch.bfloat16
-        if self.blas and bf16 and dim in (32, 64, 128) and self._flash_rows(tokens, kv_heads, group, keys):
+        if self.blas and dim in ((32, 64, 128) if bf16 else (16, 32, 64)) and self._flash_rows(tokens, kv_heads, group, keys, bf16):
             if self._flash_attention(out, q, k_past, k_new, v_past, v_new, mask, sinks, scale):
                 return out
         if self.blas and bf16 and dim % 32 == 0 and dim <= 128 and tokens >= MATRIX_ATTENTION_TOKENS:
@@ -2316,11 +2322,13 @@ class HIPCodegen(Codegen):
         return out
 
     @staticmethod
-    def _flash_rows(tokens: int, kv_heads: int, group: int, keys: int) -> bool:
-        """Whether an attention of these extents goes to ``attention_flash_bf16``: below MATRIX_ATTENTION_TOKENS queries
+    def _flash_rows(tokens: int, kv_heads: int, group: int, keys: int, bf16: bool) -> bool:
+        """Whether an attention of these extents goes to ``attention_flash``. bfloat16: below MATRIX_ATTENTION_TOKENS queries
         every one but a decode step over a long cache (one query over more than 4 decode splits of keys has kernels of
         its own); from there on those whose 16-query tiles would leave compute units idle and whose keys are enough
-        to split."""
+        to split. Float: more queries than a following few-row product could take as an epilogue."""
+        if not bf16:
+            return tokens > 16
         if tokens < MATRIX_ATTENTION_TOKENS:
             return tokens > 1 or keys <= 4 * DECODE_SPLIT_KEYS
         return keys > 4 * DECODE_SPLIT_KEYS and kv_heads * -(-tokens // 16) < MFMA_CUS
@@ -2620,12 +2628,13 @@ class HIPCodegen(Codegen):
             operands["k_past"], operands["v_past"] = (k_past, k_past.shape), (v_past, v_past.shape)
         # Check every layout before anything is stored: rows of q, K and V contiguous along the head
         # dimension with 16-byte aligned starts, unit key stride in the mask, one sink per head.
+        chunk = 16 // ITEMSIZE[q.dtype]
         for name, (value, shape) in operands.items():
             stored, strides = self._in_place(value)
             pad = len(shape) - len(value.shape)
             strides = [0] * pad + [0 if size == 1 else stride for size, stride in zip(value.shape, strides)]
             offset = stored.view.offset if stored is not None and stored.view.base is not None else 0
-            if name in ("q", "k_new", "v_new", "k_past", "v_past") and (strides[-1] != 1 or any(x % 8 for x in strides[:-1]) or offset % 8):
+            if name in ("q", "k_new", "v_new", "k_past", "v_past") and (strides[-1] != 1 or any(x % chunk for x in strides[:-1]) or offset % chunk):
                 return None
             if (name == "mask" and strides[3] != 1) or (name == "sinks" and strides[2] != 0):
                 return None
@@ -2652,7 +2661,7 @@ class HIPCodegen(Codegen):
         kp = plan["k_past"][1] if plan["k_past"] is not None else plan["k_new"][1]
         vp = plan["v_past"][1] if plan["v_past"] is not None else plan["v_new"][1]
         kn, vn = plan["k_new"][1], plan["v_new"][1]
-        k.line("chroma::AttentionOperands a;")
+        k.line("chroma::AttentionOperands a;" if out.dtype == torch.bfloat16 else f"chroma::AttentionOperandsOf<{ctype_of(out.dtype)}> a;")
         k.line(f"a.q = {pointer('q')}; a.qt = {q_strides[0]}u; a.qh = {q_strides[1]}u; a.qg = {q_strides[2]}u;")
         k.line(f"a.k_past = {pointer('k_past')}; a.k_new = {pointer('k_new')}; a.v_past = {pointer('v_past')}; a.v_new = {pointer('v_new')};")
         k.line(f"a.kpj = {kp[0]}u; a.kph = {kp[1]}u; a.knj = {kn[0]}u; a.knh = {kn[1]}u;")
@@ -2669,8 +2678,8 @@ class HIPCodegen(Codegen):
         return mantissa == 0.5 and -64 <= exponent <= 1
 
     def _flash_attention(self, out, q, k_past, k_new, v_past, v_new, mask, sinks, scale) -> bool:
-        """bfloat16 attention of few query rows on the matrix cores with the keys split over waves and workgroups
-        (``attention_flash_bf16``); False (nothing emitted) when an operand's layout or the mask does not allow it."""
+        """Attention of few query rows (or a float prefill) on the matrix cores with the keys split over waves and
+        workgroups (``attention_flash``); False (nothing emitted) when an operand's layout or the mask does not allow it."""
         tokens, kv_heads, group, dim = q.shape
         past = k_past.shape[0] if k_past is not None else 0
         keys = past + k_new.shape[0]
@@ -2680,11 +2689,13 @@ class HIPCodegen(Codegen):
         plan = self._attention_plan(q, k_past, k_new, v_past, v_new, mask, sinks)
         if plan is None:
             return False
-        tiles = 2 if tokens * group > 16 else 1  # 16-row tiles per wave: two share each K and V fragment
+        # two 16-row tiles per wave share each K and V fragment once there is a workgroup of one tile per compute unit
+        tiles = 2 if tokens * group * kv_heads > 16 * MFMA_CUS else 1
         groups = -(-tokens * group // (16 * tiles))
         blocks = -(-keys // 64)
-        # as many splits as bring the launch to one workgroup of 4 waves per compute unit, each wave a block at least
-        splits = max(1, min(-(-blocks // 4), MFMA_CUS // (kv_heads * groups)))
+        # keys are split (and the splits added by a second launch) as far as a workgroup and a half per compute unit and two
+        # blocks for every wave
+        splits = max(1, min(-(-blocks // 8), MFMA_CUS * 3 // 2 // (kv_heads * groups)))
         operands = [entry[0] for entry in plan.values() if entry is not None]
         partial = self.allocate((kv_heads * groups * splits * 16 * tiles * (dim + 2),), torch.float32) if splits > 1 else None
         k = Kernel(1)
@@ -2692,7 +2703,7 @@ class HIPCodegen(Codegen):
         self._attention_operands(k, out, plan, q, past, keys, scale)
         scratch = k.slot(partial.name, torch.float32, writable=True, extent=self.extents[partial.name]) if partial is not None else "nullptr"
         quads = not (plan["mask"][1][2] % 4 or plan["mask"][2] % 4 or keys % 4)
-        k.line(f"chroma::attention_flash_bf16<{dim}, {group}, {tiles}, {str(self._power_of_two(scale)).lower()}, {str(quads).lower()}>"
+        k.line(f"chroma::attention_flash<{ctype_of(out.dtype)}, {dim}, {group}, {tiles}, {str(self._power_of_two(scale)).lower()}, {str(quads).lower()}>"
                f"(a, {splits}u, {scratch});")
         self.launch(k, (kv_heads, groups, splits), 256, operands, kind="attention_flash")
         if partial is not None:
@@ -2701,10 +2712,11 @@ class HIPCodegen(Codegen):
             base = k.slot(value.root.name, value.root.dtype, extent=self.extents[value.root.name])
             slot = k.slot(out.name, out.dtype, writable=True, extent=self.extents[out.name])
             scratch = k.slot(partial.name, torch.float32, extent=self.extents[partial.name])
-            k.line(f"chroma::attention_flash_combine<{dim}, {group}, {tiles}>({scratch}, {base} + {offset}u, {strides[0]}u, {strides[1]}u, {slot}, {tokens}u, {splits}u);")
+            k.line(f"chroma::attention_flash_combine<{ctype_of(out.dtype)}, {dim}, {group}, {tiles}>({scratch}, {base} + {offset}u, {strides[0]}u, {strides[1]}u, "
+                   f"{slot}, {tokens}u, {splits}u);")
             self.launch(k, (kv_heads, groups, 1), 256, [partial, value], kind="attention_flash_combine")
         self.fused_attentions += 1
-        if tokens >= MATRIX_ATTENTION_TOKENS:
+        if tokens >= MATRIX_ATTENTION_TOKENS and out.dtype == torch.bfloat16:
             self.mfma_matmuls += 1
         return True
 
@@ -3066,7 +3078,12 @@ class HIPCodegen(Codegen):
         = (value, buffer) the ring body's epilogue writes ``value`` (which reads this product's output)
         into ``buffer``, and the product too unless ``store_product`` is false (``_activation_epilogue``)."""
         path, threads, width, waves, last = 1, 256, 128, 4, 128
+        split = self._kwave_experts(weight, x, tokens * selected, experts, channels, inner)
+        if split is not None:
+            return self._kwave_grouped_kernel(out, weight, indices, x, tokens, selected, experts, channels, inner, per_slot, split, activation, store_product)
         ring = next(((n, w, t) for n, w, t in RING_EXPERT_TILES if channels % n == 0), None)
+        if ring is not None and ring[0] == 320 and channels % FEW_SLOT_TILE[0] == 0 and tokens * selected <= FEW_EXPERT_SLOTS * experts:
+            ring = FEW_SLOT_TILE
         if out.dtype == torch.bfloat16 and inner % 32 == 0 and ring is not None:
             path, (width, waves, last) = 3, ring
             threads = 64 * waves
@@ -3093,9 +3110,50 @@ class HIPCodegen(Codegen):
         )
         return k, 8 * -(-(-(-channels // width) * tiles) // 8), threads, path, scratch
 
+    def _kwave_experts(self, weight: Value, x: Value, slots: int, experts: int, channels: int, inner: int) -> Optional[Tuple[int, int]]:
+        """(16-slot blocks, 16-channel blocks) of the K-split grouped body's pieces, chosen by ``_kwave_plan``'s account over
+        evenly filled experts, or None: bfloat16 products keep the ring body where it applies (GPT-OSS-20B's layer of 100
+        tokens 363 us on the ring, 376 here; 400 tokens 418 and 512: every piece starts with its own chain of routing
+        loads) and the direct ones above FEW_EXPERT_SLOTS slots an expert."""
+        size = ITEMSIZE[x.dtype]
+        if not self._kwave_fits(x, weight, slots, channels, inner) or channels % 4:
+            return None
+        if x.dtype == torch.bfloat16 and (slots > FEW_EXPERT_SLOTS * experts or inner % 32 == 0 and any(channels % n == 0 for n, _, _ in RING_EXPERT_TILES)):
+            return None
+        best, rows = None, -(-slots // experts)
+        for tm in (1, 2, 4, 8):
+            for tn in (1, 2, 3, 4, 6):
+                if tm * tn > 36 or 3 * KWAVE_WAVES * (tm + tn) << 10 > KWAVE_LDS or 16 * tm >= 2 * max(16, rows):
+                    continue
+                rounds = -(-(experts * -(-rows // (16 * tm)) * -(-channels // (16 * tn))) // MFMA_CUS)
+                load = 16 * (tm + tn) * inner * size / (KWAVE_LOAD_GBS * 1e3)
+                matrix = 2 * 256 * tm * tn * inner / (KWAVE_MATRIX_GFLOPS[x.dtype] * 1e3)
+                cost = (rounds * max(load, matrix), tm, tn)
+                best = min(best or cost, cost)
+        return best[1:]
+
+    def _kwave_grouped_kernel(self, out, weight, indices, x, tokens, selected, experts, channels, inner, per_slot, split, activation, store_product):
+        """``_grouped_kernel`` on the K-split body (path 4)."""
+        tm, tn = split
+        scratch, _ = self._route(indices, experts)
+        k = Kernel(1)
+        k.min_waves = 1
+        w, xs = self._matrix_slot(k, weight), self._matrix_slot(k, x)
+        table = k.slot(scratch.name, torch.int64, extent=self.extents[scratch.name])
+        if activation is None:
+            destination, epilogue = k.slot(out.name, out.dtype, writable=True, extent=self.extents[out.name]), ""
+        else:
+            self._emit_activation_epilogue(k, out, indices, *activation, tokens, selected, channels, store_product)
+            destination, epilogue = f"static_cast<{ctype_of(out.dtype)}*>(nullptr)", ", epilogue"
+        slots = min(4, KWAVE_LDS // (KWAVE_WAVES * (tm + tn) << 10))
+        k.line(f"chroma::grouped_expert_kwave<{ctype_of(out.dtype)}, {str(per_slot).lower()}, {tm}, {tn}, {KWAVE_WAVES}, {slots}>({w}, {xs}, {destination}, "
+               f"reinterpret_cast<const int32_t*>({table}), {tokens * selected}u, {selected}u, {experts}u, {channels}u, {inner}u{epilogue});")
+        pieces = tokens * selected // (16 * tm) + experts  # at most: an expert's last piece may be partial
+        return k, 8 * -(-(-(-channels // (16 * tn)) * pieces) // 8), 64 * KWAVE_WAVES, 4, scratch
+
     def _emit_activation_epilogue(self, k: Kernel, product: Value, indices: Value, value: Value, buffer: Value, tokens: int,
                                   selected: int, channels: int, store_product: bool) -> None:
-        """The lambda the ring body calls per (slot, 4 consecutive channels c .. c + 3) of ``product``
+        """The lambda the body calls per (slot, 4 consecutive channels c .. c + 3) of ``product``
         [tokens, selected, channels]: it rounds the four sums as the product's store would (and stores
         them when ``store_product``), then evaluates ``value`` [tokens, selected, channels / 2] at channels
         c / 2 and c / 2 + 1 (a gated activation reads channels 2i and 2i + 1 of the product for its channel
@@ -3106,13 +3164,17 @@ class HIPCodegen(Codegen):
         raises ``_NotFusible``."""
         half = channels // 2
         slot = k.slot(buffer.name, buffer.dtype, writable=True, extent=self.extents[buffer.name])
+        bf16 = product.dtype == torch.bfloat16
         with k.block("auto epilogue = [&](uint32_t slot, uint32_t column, const float* sums, uint32_t expert) {", "};"):
-            k.line("uint16_t bits[4];")
-            k.line("float u[4];")
-            k.line("for (int r = 0; r < 4; ++r) {")
-            k.line("    bits[r] = chroma::f32_to_bf16(sums[r]);")
-            k.line("    u[r] = chroma::bf16_to_f32(bits[r]);  // the product as stored")
-            k.line("}")
+            if bf16:
+                k.line("uint16_t bits[4];")
+                k.line("float u[4];")
+                k.line("for (int r = 0; r < 4; ++r) {")
+                k.line("    bits[r] = chroma::f32_to_bf16(sums[r]);")
+                k.line("    u[r] = chroma::bf16_to_f32(bits[r]);  // the product as stored")
+                k.line("}")
+            else:
+                k.line("const float u[4] = {sums[0], sums[1], sums[2], sums[3]};")
             b = Aff.of(k.atom(f"slot / {selected}u", tokens - 1, prefix="t"))
             e = Aff.of(k.atom(f"slot % {selected}u", selected - 1, prefix="t"))
             h = k.atom("column / 2u", half - 2, prefix="h")
@@ -3121,8 +3183,11 @@ class HIPCodegen(Codegen):
                 target = k.slot(product.root.name, product.dtype, writable=True, extent=self.extents[product.root.name])
                 at = row + Aff.of(h, 2) + product.view.offset
                 k.check_bounds(target, at + 3)
-                k.line(f"*reinterpret_cast<uint2*>({target} + {at.code()}) = uint2{{uint32_t(bits[0]) | (uint32_t(bits[1]) << 16), "
-                       "uint32_t(bits[2]) | (uint32_t(bits[3]) << 16)};")
+                if bf16:
+                    k.line(f"*reinterpret_cast<uint2*>({target} + {at.code()}) = uint2{{uint32_t(bits[0]) | (uint32_t(bits[1]) << 16), "
+                           "uint32_t(bits[2]) | (uint32_t(bits[3]) << 16)};")
+                else:
+                    k.line(f"*reinterpret_cast<float4*>({target} + {at.code()}) = float4{{u[0], u[1], u[2], u[3]}};")
 
             def lane_value(address: Aff) -> tuple:
                 rest = address.without(h)
@@ -3146,21 +3211,24 @@ class HIPCodegen(Codegen):
                 del k.register_reads[indices.root.name]
             at = b.scale(selected * half) + e.scale(half) + Aff.of(h)
             k.check_bounds(slot, at + 1)
-            k.line(f"*reinterpret_cast<uint32_t*>({slot} + {at.code()}) = uint32_t(chroma::f32_to_bf16({names[0]})) | "
-                   f"(uint32_t(chroma::f32_to_bf16({names[1]})) << 16);")
+            if bf16:
+                k.line(f"*reinterpret_cast<uint32_t*>({slot} + {at.code()}) = uint32_t(chroma::f32_to_bf16({names[0]})) | "
+                       f"(uint32_t(chroma::f32_to_bf16({names[1]})) << 16);")
+            else:
+                k.line(f"*reinterpret_cast<float2*>({slot} + {at.code()}) = float2{{{names[0]}, {names[1]}}};")
 
     def _activation_epilogue(self, x: Value) -> Optional[Value]:
         """Store the per-slot operand ``x`` of a second expert product from the epilogue of the first when
         ``x`` is an elementwise expression of that product's output (the gated activation) and the first
-        product is the last launch, on the ring body, with ``x`` taking channels 2i and 2i + 1 for its
-        channel i (bfloat16). The first product's launch is re-emitted with the epilogue, its output is
+        product is the last launch, on the ring or the K-split body, with ``x`` taking channels 2i and 2i + 1
+        for its channel i. The first product's launch is re-emitted with the epilogue, its output is
         never written (any other read of it fails the compile), and ``x``'s readers read the stored copy.
         Removes the activation's map launch and the round trip of the product through HBM."""
         last = self.last_grouped
-        if not ACTIVATION_EPILOGUES or last is None or last["index"] != len(self.launches) - 1 or last["path"] != 3:
+        if not ACTIVATION_EPILOGUES or last is None or last["index"] != len(self.launches) - 1 or last["path"] not in (3, 4):
             return None
         out, weight, indices, xin, tokens, selected, experts, channels, inner, per_slot = last["args"]
-        if (out.name not in self.sources.get(x.name, ()) or x.dtype != torch.bfloat16 or out.dtype != torch.bfloat16
+        if (out.name not in self.sources.get(x.name, ()) or x.dtype != out.dtype or (out.dtype != torch.bfloat16 and last["path"] != 4)
                 or tuple(x.shape) != (tokens, selected, channels // 2) or channels % 4):
             return None
         buffer = self.allocate(tuple(x.shape), x.dtype)

@@ -720,20 +720,21 @@ __device__ __forceinline__ void attention_combine(const float* partial, uint32_t
 // Operands: q [T, KV, G, D] with strides (qt, qh, qg, 1); keys and values as rows [.., KV, D] with row
 // strides (past rows [0, past), new rows [past, keys)); mask[t, j] at mask + t*mt + kv*mh + g*mg + j;
 // sinks at sinks + kv*sh + g*sg; out [T, KV, G, D] contiguous. Row strides and bases keep 16-byte alignment.
-struct AttentionOperands {
-    const uint16_t* q;
+template <class T> struct AttentionOperandsOf {
+    const T* q;
     uint32_t qt, qh, qg;
-    const uint16_t *k_past, *k_new, *v_past, *v_new;
+    const T *k_past, *k_new, *v_past, *v_new;
     uint32_t kpj, kph, knj, knh, vpj, vph, vnj, vnh;
-    const uint16_t* mask;
+    const T* mask;
     uint32_t mt, mh, mg;
-    const uint16_t* sinks;
+    const T* sinks;
     uint32_t sh, sg;
-    uint16_t* out;
+    T* out;
     uint32_t tokens, past, keys, kv_heads, group;
     float scale;
     const uint8_t* live_blocks;  // [query blocks][key blocks]: 0 where the mask is -inf throughout (or nullptr)
 };
+using AttentionOperands = AttentionOperandsOf<uint16_t>;
 
 // live_blocks[qb * key_blocks + kb] for queries [64 qb, 64 qb + 64) and keys [32 kb, 32 kb + 32) of a mask
 // shared by every head: 0 when every mask value there is -inf, 2 when every one is +0.0 (the block needs

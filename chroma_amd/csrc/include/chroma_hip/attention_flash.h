@@ -1,5 +1,5 @@
-// bfloat16 grouped-query attention with sinks for few query rows: the chain of attention.h on the matrix cores, one
-// pass over the keys, each wave on key blocks of its own.
+// Grouped-query attention with sinks for few query rows (bfloat16) and for float prefills: the chain of attention.h on
+// the matrix cores, one pass over the keys, each wave on key blocks of its own.
 //
 // The group-shared kernel (``attention_heads_mfma_bf16``) gives a workgroup 16 queries and every key; with few queries
 // the chip idles (100 queries x 8 heads: 56 workgroups), and below 16 queries most of a tile is padding. Here a tile is
@@ -12,12 +12,16 @@
 // 134 -> 5 us, 36 over 4072 (128-key windows) 848 -> 13, 100 over 1100 23 + 5 (live tiles) -> 9; a whole layer's call of
 // 400 queries over 2401 keys 208 -> 150 us (with its products), 480 over 4481 307 -> 220.
 //
+// Float products run on v_mfma_f32_16x16x4f32 (256 queries of 8 heads of 16 over 512 keys: 25 us with a wave per query
+// head on the vector units).
+//
 // Rounding: the scores, scaled scores and masked scores are rounded as attention.h says; a probability is rounded to
 // bfloat16 as exp(s - m), m a running maximum of the row, before it meets V, and the row is divided by the float sum at
 // the end (the same relative rounding of each probability as when it is divided first).
 #pragma once
 
 #include "attention.h"
+#include "kwave.h"
 
 namespace chroma {
 
@@ -40,37 +44,46 @@ struct FlashMerge {
 };
 
 // MASK4: the mask's rows, first element and key count are multiples of 4 elements, so its entries are read 4 at a time.
-template <int D, int G, int RT, bool POW2, bool MASK4>
-__device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a, uint32_t splits, float* __restrict__ partial) {
-    static_assert(D % 32 == 0 && D <= 128 && G >= 1, "head dimension and group");
+template <class T, int D, int G, int RT, bool POW2, bool MASK4>
+__device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a, uint32_t splits, float* __restrict__ partial) {
+    constexpr bool BF16 = sizeof(T) == 2;
+    constexpr uint32_t CHUNK = 16u / sizeof(T), PER_ROW = D / CHUNK;  // elements of a 16-byte chunk, chunks of a key's row
+    static_assert(PER_ROW % 4u == 0 && 64u % PER_ROW == 0 && G >= 1, "head dimension and group");
     constexpr uint32_t WAVE = 2u * kFlashKeys * D;  // LDS elements per wave: a K block and a V block
     constexpr uint32_t ROWS = 16u * RT, OPAD = D + 4u;
-    static_assert(ROWS * (OPAD + 2u) * 2u <= WAVE, "a wave's sums fit its buffers");
-    constexpr int COPIES = kFlashKeys * D / 512;   // 1 KB copies per block and operand
-    constexpr uint32_t PER_ROW = D / 8u;           // 16-byte chunks of a key's row
+    static_assert(ROWS * (OPAD + 2u) * 4u <= WAVE * sizeof(T), "a wave's sums fit its buffers");
+    constexpr int COPIES = kFlashKeys * D * sizeof(T) / 1024;  // 1 KB copies per block and operand
+    constexpr int PARTS = PER_ROW / 4u;                        // matrix-core operands of a row: 64 bytes of it each
     constexpr uint32_t SWZ = PER_ROW % 8u == 0 ? 7u : 3u;  // chunk c of row r lies at c ^ ((r / 2) & SWZ)
     constexpr float kLog2e = 1.44269504088896341f;
-    __shared__ __attribute__((aligned(1024))) uint16_t lds[kFlashWaves * WAVE];
+    __shared__ __attribute__((aligned(1024))) T lds[kFlashWaves * WAVE];
     const uint32_t lane = threadIdx.x % 64u, quad = lane / 16u, col = lane % 16u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64u);
     const uint32_t kv = blockIdx.x, row0 = blockIdx.y * ROWS, split = blockIdx.z;
     const uint32_t total_rows = a.tokens * G;
     const float neg_inf = -__builtin_inff();
-    uint16_t* ks = lds + wave * WAVE;
-    uint16_t* vs = ks + kFlashKeys * D;
+    T* ks = lds + wave * WAVE;
+    T* vs = ks + kFlashKeys * D;
 
     uint32_t query[RT];
-    bf16x8_t qf[RT][D / 32];
+    uint4 qf[RT][PARTS];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         const uint32_t row = row0 + rt * 16u + col < total_rows ? row0 + rt * 16u + col : total_rows - 1u;
         query[rt] = row / G;
 #pragma unroll
-        for (int c = 0; c < D / 32; ++c) {
-            qf[rt][c] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(a.q + size_t(query[rt]) * a.qt + kv * a.qh + (row % G) * a.qg + c * 32u + quad * 8u));
+        for (int c = 0; c < PARTS; ++c) {
+            qf[rt][c] = *reinterpret_cast<const uint4*>(a.q + size_t(query[rt]) * a.qt + kv * a.qh + (row % G) * a.qg + (c * 4u + quad) * CHUNK);
         }
     }
 
+    auto minus_infinity = [](T v) {
+        if constexpr (BF16) {
+            return v == 0xff80u;
+        } else {
+            return v == -__builtin_inff();
+        }
+    };
     // This wave's key blocks: split * 4 + wave, then every 4 * splits. With more than one, those that a mask entry of
     // this group's queries leaves alive are found first (a bit each; past 64 they all count as alive).
     const uint32_t blocks = (a.keys + kFlashKeys - 1u) / kFlashKeys, stride = kFlashWaves * splits, first = split * kFlashWaves + wave;
@@ -81,7 +94,7 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
         const uint32_t q_first = row0 / G, q_last = (row0 + ROWS < total_rows ? row0 + ROWS - 1u : total_rows - 1u) / G;
         alive = 0ull;
         for (uint32_t n0 = 0; n0 < (mine < 64u ? mine : 64u); n0 += 4u) {
-            uint16_t bits[4][TQ];
+            T bits[4][TQ];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t j = (first + (n0 + i) * stride) * kFlashKeys + lane;
@@ -96,7 +109,7 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
                 bool any = false;
 #pragma unroll
                 for (int t = 0; t < TQ; ++t) {
-                    any |= bits[i][t] != 0xff80u;
+                    any |= !minus_infinity(bits[i][t]);
                 }
                 any = any && n0 + i < mine && (first + (n0 + i) * stride) * kFlashKeys + lane < a.keys;
                 if (__ballot(any) != 0ull) {
@@ -113,14 +126,14 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
     };
 
     // Copies: lane l moves position l % PER_ROW of row l / PER_ROW of each 1 KB piece. Keys past the end repeat the last.
-    auto copy = [&](uint16_t* to, const uint16_t* past, uint32_t pj, uint32_t ph, const uint16_t* fresh, uint32_t nj, uint32_t nh, uint32_t block) {
+    auto copy = [&](T* to, const T* past, uint32_t pj, uint32_t ph, const T* fresh, uint32_t nj, uint32_t nh, uint32_t block) {
 #pragma unroll
         for (int i = 0; i < COPIES; ++i) {
             const uint32_t r = i * (64u / PER_ROW) + lane / PER_ROW, chunk = (lane % PER_ROW) ^ ((r / 2u) & SWZ);
             const uint32_t j = block * kFlashKeys + r < a.keys ? block * kFlashKeys + r : a.keys - 1u;
             const bool old = j < a.past;
-            const uint16_t* row = old ? past + (size_t(j) * pj + kv * ph) : fresh + (size_t(j - a.past) * nj + kv * nh);
-            __builtin_amdgcn_global_load_lds((global_void*)(row + chunk * 8u), (lds_void*)(to + i * 512u), 16, 0, 0);
+            const T* row = old ? past + (size_t(j) * pj + kv * ph) : fresh + (size_t(j - a.past) * nj + kv * nh);
+            __builtin_amdgcn_global_load_lds((global_void*)(row + chunk * CHUNK), (lds_void*)(to + i * (1024u / sizeof(T))), 16, 0, 0);
         }
     };
     auto copy_k = [&](uint32_t block) { copy(ks, a.k_past, a.kpj, a.kph, a.k_new, a.knj, a.knh, block); };
@@ -146,20 +159,21 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
         const uint32_t block = first + n * stride, next = next_of(n + 1u);
         // mask entries of this lane: keys 16 t + 4 quad .. + 3 of the block, its query
         // (every load unconditional, clamped: a guarded load would end its branch with a wait)
-        uint2 m[RT][4];
-        uint16_t element[RT][4][4];
+        struct alignas(4 * sizeof(T)) Four {
+            T v[4];
+        } m[RT][4];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const uint32_t j = block * kFlashKeys + t * 16u + quad * 4u;
-                const uint16_t* row = a.mask + size_t(query[rt]) * a.mt;
+                const T* row = a.mask + size_t(query[rt]) * a.mt;
                 if constexpr (MASK4) {
-                    m[rt][t] = *reinterpret_cast<const uint2*>(row + (j < a.keys ? j : a.keys - 4u));
+                    m[rt][t] = *reinterpret_cast<const Four*>(row + (j < a.keys ? j : a.keys - 4u));
                 } else {
 #pragma unroll
                     for (uint32_t r = 0; r < 4u; ++r) {
-                        element[rt][t][r] = row[j + r < a.keys ? j + r : a.keys - 1u];
+                        m[rt][t].v[r] = row[j + r < a.keys ? j + r : a.keys - 1u];
                     }
                 }
             }
@@ -175,49 +189,43 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 s[rt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                const uint32_t j = block * kFlashKeys + t * 16u + quad * 4u;
-                if constexpr (!MASK4) {
-                    uint32_t e[4];
-#pragma unroll
-                    for (uint32_t r = 0; r < 4u; ++r) {
-                        e[r] = j + r < a.keys ? uint32_t(element[rt][t][r]) : 0xff80u;
-                    }
-                    m[rt][t] = uint2{e[0] | e[1] << 16, e[2] | e[3] << 16};
-                } else if (j >= a.keys) {
-                    m[rt][t] = uint2{0xff80ff80u, 0xff80ff80u};
-                }
             }
 #pragma unroll
-            for (int c = 0; c < D / 32; ++c) {
+            for (int c = 0; c < PARTS; ++c) {
                 const uint32_t r = t * 16u + col;
-                const bf16x8_t kf = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(ks + r * D + ((c * 4u + quad) ^ ((r / 2u) & SWZ)) * 8u));
+                const uint4 kf = *reinterpret_cast<const uint4*>(ks + r * D + ((c * 4u + quad) ^ ((r / 2u) & SWZ)) * CHUNK);
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
-                    s[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][c], s[rt], 0, 0, 0);
+                    kwave_mfma<T>(kf, qf[rt][c], s[rt]);
                 }
             }
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
                 for (int r = 0; r < 4; r += 2) {
+                    const bool in_x = block * kFlashKeys + t * 16u + quad * 4u + r < a.keys, in_y = block * kFlashKeys + t * 16u + quad * 4u + r + 1u < a.keys;
+                    const float mx = in_x ? widen_of<T>(m[rt][t].v[r]) : neg_inf, my = in_y ? widen_of<T>(m[rt][t].v[r + 1]) : neg_inf;
                     float x = s[rt][r], y = s[rt][r + 1];
-                    round_bf16_pair(x, y);
-                    x *= a.scale;
-                    y *= a.scale;
-                    if constexpr (!POW2) {
+                    if constexpr (BF16) {
                         round_bf16_pair(x, y);
                     }
-                    const uint32_t w = r == 0 ? m[rt][t].x : m[rt][t].y;
-                    x += __uint_as_float(w << 16);
-                    y += __uint_as_float(w & 0xffff0000u);
-                    round_bf16_pair(x, y);
+                    x *= a.scale;
+                    y *= a.scale;
+                    if constexpr (BF16 && !POW2) {
+                        round_bf16_pair(x, y);
+                    }
+                    x += mx;
+                    y += my;
+                    if constexpr (BF16) {
+                        round_bf16_pair(x, y);
+                    }
                     u[rt][t][r] = x;
                     u[rt][t][r + 1] = y;
                 }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        bf16x8_t pf[RT][2];
+        bf16x8_t pf[RT][2];  // bfloat16: probabilities of the products' operands; float ones replace u
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             float top = neg_inf;
@@ -248,15 +256,21 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
                 }
 #pragma unroll
                 for (int r = 0; r < 4; r += 2) {
-                    const bf16x2_t pair = __builtin_convertvector(f32x2_t{e[r], e[r + 1]}, bf16x2_t);
-                    pf[rt][t / 2][t % 2 * 4 + r] = pair[0];
-                    pf[rt][t / 2][t % 2 * 4 + r + 1] = pair[1];
+                    if constexpr (BF16) {
+                        const bf16x2_t pair = __builtin_convertvector(f32x2_t{e[r], e[r + 1]}, bf16x2_t);
+                        pf[rt][t / 2][t % 2 * 4 + r] = pair[0];
+                        pf[rt][t / 2][t % 2 * 4 + r + 1] = pair[1];
+                    } else {
+                        u[rt][t][r] = e[r];
+                        u[rt][t][r + 1] = e[r + 1];
+                    }
                 }
             }
         }
         // slots 0-3 and 4-7 of lane (d, quad) hold keys 32 h + 4 quad + r and 32 h + 16 + 4 quad + r: one transposing
         // read each (lane 4 r + c of a quad gives the address of key r's columns 4 c .. + 3 and receives column
         // 4 r + c of the four keys)
+        if constexpr (BF16) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
@@ -273,6 +287,24 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
                     o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[rt][h], o[rt][dt], 0, 0, 0);
+                }
+            }
+        }
+        } else {
+            // product (t, r) takes keys 16 t + 4 quad + r: this lane's own probability, V's element (key, d = 16 dt + col)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t key = t * 16u + quad * 4u + r;
+#pragma unroll
+                    for (int dt = 0; dt < D / 16; ++dt) {
+                        const float v = vs[key * D + ((dt * 4u + col / 4u) ^ ((key / 2u) & SWZ)) * 4u + col % 4u];
+#pragma unroll
+                        for (int rt = 0; rt < RT; ++rt) {
+                            o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, u[rt][t][r], o[rt][dt], 0, 0, 0);
+                        }
+                    }
                 }
             }
         }
@@ -304,13 +336,13 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
     }
     __syncthreads();
     const float* parts = reinterpret_cast<const float*>(lds);
-    constexpr uint32_t PART = WAVE / 2u;  // floats of a wave's buffers
+    constexpr uint32_t PART = WAVE * sizeof(T) / 4u;  // floats of a wave's buffers
     for (uint32_t i = threadIdx.x; i < ROWS * (D / 4u); i += 64u * kFlashWaves) {
         const uint32_t r = i / (D / 4u), d = i % (D / 4u) * 4u, row = row0 + r;
         if (row >= total_rows) {
             continue;
         }
-        FlashMerge merge{splits == 1u ? bf16_to_f32(a.sinks[kv * a.sh + (row % G) * a.sg]) : neg_inf, 0.0f};
+        FlashMerge merge{splits == 1u ? widen_of<T>(a.sinks[kv * a.sh + (row % G) * a.sg]) : neg_inf, 0.0f};
         const float sink = merge.top;
 #pragma unroll
         for (uint32_t w = 0; w < kFlashWaves; ++w) {
@@ -326,9 +358,8 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
         if (splits == 1u) {
             merge.total += merge.weight(sink);
             sum *= 1.0f / merge.total;
-            uint16_t* to = a.out + ((size_t(row / G) * a.kv_heads + kv) * G + row % G) * D + d;
-            *reinterpret_cast<uint2*>(to) = uint2{uint32_t(f32_to_bf16(sum[0])) | uint32_t(f32_to_bf16(sum[1])) << 16,
-                                                  uint32_t(f32_to_bf16(sum[2])) | uint32_t(f32_to_bf16(sum[3])) << 16};
+            const float y[4] = {sum[0], sum[1], sum[2], sum[3]};
+            kwave_store<T>(a.out + ((size_t(row / G) * a.kv_heads + kv) * G + row % G) * D + d, y, d, D);
         } else {
             float* to = partial + size_t((kv * gridDim.y + blockIdx.y) * splits + split) * flash_partial_floats<D, RT>();
             *reinterpret_cast<f32x4_t*>(to + 2u * ROWS + r * D + d) = sum;
@@ -341,9 +372,9 @@ __device__ __forceinline__ void attention_flash_bf16(const AttentionOperands& a,
 }
 
 // The splits of every row, in order, and the sink (grid: KV heads x row groups, 256 threads).
-template <int D, int G, int RT>
-__device__ __forceinline__ void attention_flash_combine(const float* __restrict__ partial, const uint16_t* __restrict__ sinks, uint32_t sh,
-                                                        uint32_t sg, uint16_t* __restrict__ out, uint32_t tokens, uint32_t splits) {
+template <class T, int D, int G, int RT>
+__device__ __forceinline__ void attention_flash_combine(const float* __restrict__ partial, const T* __restrict__ sinks, uint32_t sh,
+                                                        uint32_t sg, T* __restrict__ out, uint32_t tokens, uint32_t splits) {
     constexpr uint32_t ROWS = 16u * RT, PART = flash_partial_floats<D, RT>();
     const uint32_t kv = blockIdx.x, row0 = blockIdx.y * ROWS;
     const float* parts = partial + size_t(kv * gridDim.y + blockIdx.y) * splits * PART;
@@ -352,7 +383,7 @@ __device__ __forceinline__ void attention_flash_combine(const float* __restrict_
         if (row >= tokens * G) {
             continue;
         }
-        const float sink = bf16_to_f32(sinks[kv * sh + (row % G) * sg]);
+        const float sink = widen_of<T>(sinks[kv * sh + (row % G) * sg]);
         FlashMerge merge{sink, 0.0f};
         for (uint32_t s = 0; s < splits; ++s) {
             merge.top = __builtin_fmaxf(merge.top, parts[s * PART + 2u * r]);
@@ -365,9 +396,8 @@ __device__ __forceinline__ void attention_flash_combine(const float* __restrict_
         }
         merge.total += merge.weight(sink);
         sum *= 1.0f / merge.total;
-        uint16_t* to = out + ((size_t(row / G) * gridDim.x + kv) * G + row % G) * D + d;
-        *reinterpret_cast<uint2*>(to) = uint2{uint32_t(f32_to_bf16(sum[0])) | uint32_t(f32_to_bf16(sum[1])) << 16,
-                                              uint32_t(f32_to_bf16(sum[2])) | uint32_t(f32_to_bf16(sum[3])) << 16};
+        const float y[4] = {sum[0], sum[1], sum[2], sum[3]};
+        kwave_store<T>(out + ((size_t(row / G) * gridDim.x + kv) * G + row % G) * D + d, y, d, D);
     }
 }
 

@@ -109,8 +109,64 @@ def test_few_query_attention(tmp_path, tokens, past, kv_heads, group, dim, windo
     inputs = attention_inputs(tokens, past, kv_heads, group, dim, window)
     exported = torch.export.export(SinkAttention(), inputs)
     with chroma_amd.compile(exported, tmp_path / "hip") as model:
-        assert "attention_flash_bf16" in (tmp_path / "hip" / "model.hip").read_text()
+        assert "attention_flash<" in (tmp_path / "hip" / "model.hip").read_text()
         got = [model(*inputs) for _ in range(2)]
     want = compile_cpu(exported, tmp_path / "cpu")(*[numpy_of(v) for v in inputs])
     for result in got:
         assert_close(result, want, rtol=2e-2, atol=1e-2)
+
+
+class GroupedExperts(torch.nn.Module):
+    def forward(self, weights, indices, x, per_slot):
+        selected = weights[indices]
+        return torch.einsum("beck,bk->bec", selected, x), torch.einsum("beck,bek->bec", selected, per_slot)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("experts, channels, inner, counts", [
+    (3, 100, 136, [1, 63, 0]),          # one slot, an empty expert, K and channels inside a tile
+    (12, 256, 128, [16, 17, 32, 33, 64, 65, 1, 0, 0, 28, 60, 4]),  # every count of live 16-row blocks
+    (70, 36, 264, [2] * 64 + [0] * 5 + [64]),  # more experts than lanes
+])
+def test_k_split_expert_products(tmp_path, dtype, experts, channels, inner, counts):
+    generator = torch.Generator().manual_seed(sum(counts) + channels)
+    slots = torch.cat([torch.full((count,), e, dtype=torch.int64) for e, count in enumerate(counts)])
+    slots = slots[torch.randperm(len(slots), generator=generator)]
+    selected = 4 if len(slots) % 4 == 0 else 1
+    indices = slots.reshape(-1, selected)
+    indices[0, 0] -= experts  # ids wrap when negative
+    weights = (torch.randn(experts, channels, inner, generator=generator) * 0.05).to(dtype)
+    x = torch.randn(len(indices), inner, generator=generator).to(dtype)
+    per_slot = torch.randn(*indices.shape, inner, generator=generator).to(dtype)
+    exported = export(GroupedExperts(), weights, indices, x, per_slot)
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        assert (tmp_path / "hip" / "model.hip").read_text().count("grouped_expert_kwave") == 2
+        up, down = model(weights, indices, x, per_slot)
+        bad = indices.clone()
+        bad[-1, -1] = experts
+        with pytest.raises(IndexError):
+            model(weights, bad, x, per_slot)
+    w = weights.double()[indices]
+    assert_sums(up, torch.einsum("beck,bk->bec", w, x.double()), inner, 0.05, dtype)
+    assert_sums(down, torch.einsum("beck,bek->bec", w, per_slot.double()), inner, 0.05, dtype)
+
+
+@pytest.mark.gpu
+def test_float_activation_epilogue_is_bit_identical(tmp_path, monkeypatch):
+    """The float MoE MLP whose clamped SwiGLU is written by its up product's epilogue against the build with a separate
+    launch, bit for bit, with the product returned or not."""
+    from chroma_amd._src.codegen import hip as codegen
+    from tests.helpers import ExpertMLP, leaves
+
+    x = torch.randn(96, 128, generator=torch.Generator().manual_seed(3)) * 2
+    for product in (False, True):
+        exported = torch.export.export(ExpertMLP(128, 64, seed=1, std=0.08, product=product).float().eval(), (x,))
+        runs = []
+        for fused in (False, True):
+            monkeypatch.setattr(codegen, "ACTIVATION_EPILOGUES", fused)
+            with chroma_amd.compile(exported, tmp_path / f"{product}{fused}") as program:
+                assert program.stats["expert_epilogues"] == int(fused)
+                runs.append([np.asarray(a).copy() for a in leaves(program(x))])
+        for plain, fused in zip(*runs):
+            np.testing.assert_array_equal(fused, plain)
