@@ -100,6 +100,16 @@ KWAVE_LOAD_GBS = 53.0
 KWAVE_MATRIX_GFLOPS = {torch.float32: 480.0, torch.bfloat16: 5000.0}
 KWAVE_PREFETCH = (512, 8 << 20)  # rows from which, and weight bytes up to which, its weights are still read ahead
 KWAVE_LDS = 147 << 10  # bytes of LDS a workgroup's rings take at most
+# The weight-streaming body by such an account: its launch and prologue, W's bytes, and per row of X and million elements
+# of W. Measured with X behind an RMSNorm unless marked (microseconds at 2 / 4 / 8 / 16 rows, K-split body in parentheses):
+# bfloat16 2880 -> 5120 13 / 22 / 58 / - (12.6-14.1), 4096 -> 2880 stored X 8 / 13 / 28 / - (6.5-7.2), 1024 -> 4096 5.8 / 7.2 /
+# 10.9 / 23 (7.6-8.0); float 1024 -> 4096 6.5 / 7.4 / 10.5 / 21 (8.9-9.3), 4096 -> 1024 SiLU product 7 / 9 / 13.6 / - (13.5),
+# 128 -> 201088 22 / 26 / 27 / 43 (34.6).
+STREAM_OVERHEAD_US = 3.0
+STREAM_GBS = 5500.0
+STREAM_ROW_US = {torch.bfloat16: 0.25, torch.float32: 0.15}
+STREAM_KWAVE_BYTES = 2 << 10
+STORE_LAUNCH_US = 2.5
 # The tiled bodies by the same account: (rows, columns) of a tile, and the load rate they reach when every compute unit
 # has a tile (600 x 2880 x 4096 on 128 x 192 57 us, 700 x 11520 x 2880 89 us; 2048 x 5120 x 2880 on 256 x 192 66-82 us).
 TILED_LOAD_GBS = {(256, 192): 36.0, (128, 192): 44.0}
@@ -427,6 +437,10 @@ class HIPCodegen(Codegen):
             return None
         out, x, weight, epsilon = last["args"]
         sources = self.sources.get(value.name, frozenset())
+        if any(self.materialized.get(name) is out for name in self.pending_of.get(value.name, frozenset())):
+            # ``value`` reads a deferred norm that has just been stored: what it reads is the norm's output, and nothing but
+            # what the norm kernel reads itself
+            sources = (sources - self.sources.get(x.name, frozenset()) - self.sources.get(weight.name, frozenset())) | {out.name}
         if (out.name not in sources or tuple(value.shape) != tuple(out.shape)
                 or any(self.binding_of(b).kind not in ("weight", "input") for b in sources if b != out.name)):
             return None
@@ -487,10 +501,43 @@ class HIPCodegen(Codegen):
             self.materialized[key] = out
         return self.materialized[key]
 
+    @staticmethod
+    def _viewed_strides(shape: Sequence[int], strides: Sequence[int], wanted: Sequence[int]) -> Optional[List[int]]:
+        """Element strides of ``wanted`` over storage laid out as (shape, strides), or None when it needs a copy: runs of
+        dimensions that lie like one (each stride the next one's stride times its extent) are split or joined freely."""
+        runs: List[Tuple[int, int]] = []  # (elements, innermost stride), outermost first
+        for size, stride in zip(shape, strides):
+            if size == 1:
+                continue
+            if runs and runs[-1][1] == size * stride:
+                runs[-1] = (runs[-1][0] * size, stride)
+            else:
+                runs.append((size, stride))
+        result: List[int] = []
+        left, stride = 1, 1
+        for size in reversed(wanted):
+            if size > 1 and left == 1:
+                if not runs:
+                    return None
+                left, stride = runs.pop()
+            if left % size:
+                return None
+            result.append(stride)
+            left //= size
+            stride *= size
+        return None if runs or left != 1 else result[::-1]
+
     def reshape(self, meta: torch.Tensor, x: Value) -> Value:
         if self.is_contiguous(x):
             return self.alias(meta, x.root, x.view.offset)
         shape = tuple(meta.shape)
+        if x.view is not None and x.view.base is not None:
+            # a strided view whose dimensions split or join in place (the heads of a row of q, k or v) stays one
+            mapping = self._viewed_strides(x.shape, x.view.strides, shape)
+            if mapping is not None:
+                result = self.reindex(meta, x.root, mapping, x.view.offset)
+                result.view = View(x.root, tuple(mapping), x.view.offset)
+                return result
 
         def closure(k: Kernel, coords: List[Aff]) -> tuple:
             return self.read_flat(k, x, Kernel.flatten(coords, shape))
@@ -671,6 +718,14 @@ class HIPCodegen(Codegen):
     def output(self, index: int, value: Value) -> None:
         if value.stored and value.root.name in self.pending_stores:
             self._flush_store(value.root.name)
+        if not value.stored and value.name in self.materialized and value.name not in self.pending_norms:
+            value = self.materialized[value.name]  # stored for an earlier reader: that copy becomes the output
+            if value.root.name in self.pending_stores:
+                self._flush_store(value.root.name)
+        root = value.root
+        if (root is not value and value.stored and root.name in self.allocations and value.view.offset == 0 and self.is_contiguous(value)
+                and root.dtype == value.dtype and math.prod(root.shape) == math.prod(value.shape)):
+            value = root  # the whole of an arena buffer under another shape
         if self.promote_output(index, value):
             return
         name = f"output{index}"
@@ -1980,6 +2035,15 @@ class HIPCodegen(Codegen):
         if self.blas and rows <= 16 and self._attention_epilogue(out, x, weight, bias, rows, columns, inner):
             self.skinny_matmuls += 1
             return out
+        if self.blas and 1 < rows <= 16 and columns > NARROW_COLUMNS and self._kwave_few_rows(x, weight, rows, columns, inner):
+            for name in sorted(self.pending_of.get(x.name, frozenset())):
+                if name not in self.materialized:
+                    self._force_norm(name)  # its kernel then writes X, when X is the norm or its cast
+            x = self.contiguous(self.store(x))
+            _, tm, tn = self._kwave_plan(rows, columns, inner, meta.dtype)
+            self._kwave_linear(out, x, weight, bias, rows, columns, inner, tm, tn)
+            self.skinny_matmuls += 1
+            return out
         plan = self._stream_plan(rows, inner, meta.dtype, columns * inner * ITEMSIZE[meta.dtype])
         if (self.blas and rows <= 16 and plan is not None and rows * inner <= LINEAR_STAGED_FLOATS
                 and weight.view.offset % (16 // ITEMSIZE[weight.dtype]) == 0):
@@ -2151,6 +2215,18 @@ class HIPCodegen(Codegen):
         chunk, size = 16 // ITEMSIZE[x.dtype], ITEMSIZE[x.dtype]
         return (inner % chunk == 0 and inner * size >= 64 * KWAVE_WAVES and x.view.offset % chunk == 0 and weight.view.offset % chunk == 0
                 and max(rows, 128) * inner * size < 2**31)
+
+    def _kwave_few_rows(self, x: Value, weight: Value, rows: int, columns: int, inner: int) -> bool:
+        """Whether a product of 2-16 rows goes to the K-split body instead of the weight-streaming one, whose time grows
+        with rows x columns x K (each lane multiplies every row; every workgroup stages all of X): by its account at
+        STREAM_OVERHEAD_US against ``_kwave_plan``'s, plus a launch that stores X when X is an expression. Only rows of
+        STREAM_KWAVE_BYTES or more: the short rows of a vocabulary product stream faster up to 12 of them."""
+        size = ITEMSIZE[x.dtype]
+        if (x.dtype not in STREAM_ROW_US or inner * size < STREAM_KWAVE_BYTES or (x.stored and not self._kwave_fits(x, weight, rows, columns, inner))
+                or inner % (16 // size) or weight.view.offset % (16 // size)):
+            return False
+        stream = STREAM_OVERHEAD_US + columns * inner * (size / (STREAM_GBS * 1e3) + rows * STREAM_ROW_US[x.dtype] * 1e-6)
+        return self._kwave_plan(rows, columns, inner, x.dtype)[0] + (0.0 if x.stored else STORE_LAUNCH_US) < stream
 
     @staticmethod
     def _kwave_plan(rows: int, columns: int, inner: int, dtype: torch.dtype) -> Tuple[float, int, int]:

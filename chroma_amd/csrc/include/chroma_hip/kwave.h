@@ -30,6 +30,8 @@ __device__ __forceinline__ void kwave_mfma(const uint4& b, const uint4& a, f32x4
     }
 }
 
+constexpr uint32_t kKwaveFlush = 4;
+
 // Elements of the LDS array: S units of TM + TN 16-row blocks (1 KiB each) per wave; a wave's partial sums (TM TN
 // KiB) take the place of its own ring.
 template <int TM, int TN, int NW, int S>
@@ -91,12 +93,32 @@ __device__ __forceinline__ void kwave_tile(const char* __restrict__ a, const uin
             copy(begin + uint32_t(n));
         }
     });
+    // Float sums of long rows are kept in two levels, kKwaveFlush units at a time, so their rounding errors grow with the
+    // root of a level's length and not of the whole (3 x 2880 x 11520: 6.2e-7 relative in one level).
+    constexpr bool LEVELS = sizeof(T) == 4;
+    f32x4_t sums[LEVELS ? TM : 1][LEVELS ? TN : 1];
+    if constexpr (LEVELS) {
+        unroll<TM>([&](auto i) { unroll<TN>([&](auto j) { sums[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}; }); });
+    }
+    auto level = [&](uint32_t u) {
+        if constexpr (LEVELS) {
+            if ((u - begin) % kKwaveFlush == kKwaveFlush - 1u || u + 1u == end) {
+                unroll<TM>([&](auto i) {
+                    unroll<TN>([&](auto j) {
+                        sums[i][j] += acc[i][j];
+                        acc[i][j] = u + 1u == end ? sums[i][j] : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    });
+                });
+            }
+        }
+    };
     uint32_t u = begin;
     for (; u + (S - 1) < end; ++u) {
         __builtin_amdgcn_s_waitcnt(vmcnt_wait((S - 2) * PER));  // unit u landed; the S - 2 after it may be in flight
         __builtin_amdgcn_sched_barrier(0);
         copy(u + (S - 1));  // into the slot unit u - 1 was read from
         multiply(u);
+        level(u);
         __builtin_amdgcn_sched_barrier(0);
     }
     unroll<S - 1>([&](auto n) {
@@ -105,6 +127,7 @@ __device__ __forceinline__ void kwave_tile(const char* __restrict__ a, const uin
             __builtin_amdgcn_s_waitcnt(vmcnt_wait(left * PER));
             __builtin_amdgcn_sched_barrier(0);
             multiply(u);
+            level(u);
             __builtin_amdgcn_sched_barrier(0);
             ++u;
         }

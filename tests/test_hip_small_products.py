@@ -170,3 +170,90 @@ def test_float_activation_epilogue_is_bit_identical(tmp_path, monkeypatch):
                 runs.append([np.asarray(a).copy() for a in leaves(program(x))])
         for plain, fused in zip(*runs):
             np.testing.assert_array_equal(fused, plain)
+
+
+def test_strides_of_views_match_numpy():
+    """``_viewed_strides`` against numpy's own reshaping in place, over random slices and orders of up to 4 dimensions."""
+    import itertools
+    import random
+
+    rng = random.Random(0)
+    in_place = copies = 0
+    for _ in range(3000):
+        a = np.arange(rng.choice([24, 96, 144])).reshape(rng.choice([(2, 3, 4, -1), (4, -1), (6, 1, -1), (-1,)]))
+        order = list(range(a.ndim))
+        if rng.random() < 0.3:
+            rng.shuffle(order)
+        view = a.transpose(order)
+        view = view[tuple(slice(rng.randint(0, 1) if s > 1 else 0, s, rng.choice([1, 1, 2])) for s in view.shape)]
+        wanted, left = [], view.size
+        while left > 1:
+            wanted.append(rng.choice([d for d in range(2, left + 1) if left % d == 0]))
+            left //= wanted[-1]
+            if rng.random() < 0.2:
+                wanted.append(1)
+        strides = HIPCodegen._viewed_strides(view.shape, [s // a.itemsize for s in view.strides], wanted)
+        if strides is None:
+            shaped = view.view()
+            with pytest.raises(AttributeError):
+                shaped.shape = tuple(wanted)
+            copies += 1
+            continue
+        start = (view.__array_interface__["data"][0] - a.__array_interface__["data"][0]) // a.itemsize
+        at = [start + sum(i * s for i, s in zip(c, strides)) for c in itertools.product(*map(range, wanted))]
+        np.testing.assert_array_equal(a.reshape(-1)[at], view.reshape(-1))
+        in_place += 1
+    assert in_place > 500 and copies > 500
+
+
+def test_outputs_take_over_stored_copies():
+    """A value stored for a kernel is not evaluated again for the output that returns it, also under another shape; a
+    buffer that two outputs return is copied for the second; a strided view is copied once."""
+    class Views(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.w = torch.nn.Parameter(torch.ones(64, 64), requires_grad=False)
+
+        def forward(self, x):
+            y = torch.nn.functional.linear(x, self.w)
+            half = y[:, 32:].contiguous().view(40, 4, 8)
+            return torch.nn.functional.linear(y * 2, self.w), y.view(40, 8, 8), y, half
+
+    generated = lower_program(export(Views(), torch.ones(40, 64)), HIPCodegen())
+    kinds = [line.split()[1].rsplit("_", 1)[0] for line in generated.files["model.plan"].splitlines() if line.startswith("launch ")]
+    # product, y * 2, product; a copy of y for the second output of the same buffer and of the strided half
+    assert kinds.count("chroma_linear_kwave") == 2 and len(kinds) == 5, kinds
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [2, 5, 16])
+def test_few_row_product_behind_a_norm(tmp_path, dtype, rows):
+    """A norm over few rows feeding a K-split product (stored by the norm kernel, in bfloat16 as its cast), a strided half of
+    the product viewed as heads, and the norm itself, against eager torch in 64 bits at the stored type's rounding."""
+    class Block(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            generator = torch.Generator().manual_seed(5)
+            self.scale = torch.nn.Parameter(1 + 0.1 * torch.randn(2048, generator=generator), requires_grad=False)
+            self.w = torch.nn.Parameter((torch.randn(4096, 2048, generator=generator) * 0.05).to(dtype), requires_grad=False)
+
+        def forward(self, x):
+            h = x.float()
+            h = (h * torch.rsqrt(torch.mean(h**2, dim=-1, keepdim=True) + 1e-5) * self.scale).to(x.dtype)
+            y = torch.nn.functional.linear(h, self.w)
+            return y, y[:, 1024:3072].contiguous().view(-1, 32, 64), h
+
+    block = Block()
+    x = torch.randn(rows, 2048, generator=torch.Generator().manual_seed(rows)).to(dtype)
+    exported = export(block, x)
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        source = (tmp_path / "hip" / "model.hip").read_text()
+        assert ("kwave_linear" in source) == (dtype == torch.bfloat16 or rows > 2)
+        got, half, normed = (as_float(a).astype(np.float64) for a in model(x))
+    wide = x.double()
+    h = wide * torch.rsqrt(torch.mean(wide**2, dim=-1, keepdim=True) + 1e-5) * block.scale.double()
+    spacing = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-21  # the norm's own float steps in float
+    np.testing.assert_allclose(normed, h.numpy(), rtol=spacing, atol=1e-30)
+    assert_sums(got.astype(np.float32), torch.from_numpy(normed) @ block.w.double().T, 2048, 0.05, dtype)
+    np.testing.assert_array_equal(half, got[:, 1024:3072].reshape(rows, 32, 64))
