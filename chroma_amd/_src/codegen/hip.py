@@ -2423,7 +2423,7 @@ class HIPCodegen(Codegen):
             ctype, inner, columns = ctype_of(out.dtype), group * dim, weight.shape[0]
             prelude.append(lambda k: f"__shared__ float attention_row[{inner}];")
             store_extra = [f"attention_row[g * {dim}u + d] = chroma::storage_round<{str(bf16).lower()}>(value);"]
-        k, _, _ = self._attention_kernel(out, q, k_past, k_new, v_past, v_new, mask, sinks, None, prelude=prelude, store_extra=store_extra)
+        k, _, _ = self._attention_kernel(out, q, k_past, k_new, v_past, v_new, mask, sinks, None, prelude=prelude, store_extra=store_extra, threads=64 * group)
         # A small W is requested before the attention, so its round trip overlaps the attention's own loads;
         # a large one once the attention is done (loads complete in order, see _stream_linear)
         early = epilogue is not None and columns * inner * ITEMSIZE[weight.dtype] <= EARLY_FETCH_BYTES
@@ -2560,14 +2560,16 @@ class HIPCodegen(Codegen):
 
     def _attention_kernel(self, out, q, k_past, k_new, v_past, v_new, mask, sinks, split, loaders: bool = True,
                           prelude: Sequence = (), fresh: Optional[Tuple[Tuple[str, ...], str]] = None,
-                          store_extra: Sequence[str] = ()) -> Tuple[Kernel, str, str]:
+                          store_extra: Sequence[str] = (), threads: int = 0) -> Tuple[Kernel, str, str]:
         """A kernel over (query row, key/value head) with the attention loaders and the result store
         declared as lambdas (operands read through generated code, so views and fused expressions are
         evaluated in place); returns it with the C expression of its ``AttentionSplit`` and the C
         expression of its first split row in the split scratch. ``prelude`` lines open the kernel;
         ``fresh`` = (key sources, C condition) stages only those sources' new rows, and only in workgroups
-        where the condition holds (no ``load_k``/``load_v`` lambdas are declared then)."""
+        where the condition holds (no ``load_k``/``load_v`` lambdas are declared then). ``threads`` (the workgroup's, when
+        given) places the staging of the new rows behind the threads that stage q."""
         tokens, kv_heads, group, dim = q.shape
+        staging_from = [group * dim if threads else 0]  # the first thread of the next staging loop
         past = k_past.shape[0] if k_past is not None else 0
         keys = past + k_new.shape[0]
         k = Kernel(1)
@@ -2610,22 +2612,26 @@ class HIPCodegen(Codegen):
                 # cooperatively, into LDS; the key loops then read plain LDS values.
                 k.line(f"__shared__ float {name}_new[{fresh * dim}];")
                 with k.block(f"if ({fresh_only[1]}) {{" if fresh_only is not None else "{"):
-                    # Runs of 32 elements, one per wave (its other 32 lanes idle): with head dimensions of 64
-                    # or more, each half of a head's row (the two sides of a rotary embedding) is evaluated
-                    # by whole waves, without diverging.
-                    runs = -(-fresh * dim // 32)
-                    with k.block(f"for (uint32_t slot = threadIdx.x; slot < {runs * 64}u; slot += blockDim.x) {{"):
-                        k.line("const uint32_t i = slot / 64u * 32u + slot % 64u;")
-                        with k.block(f"if (slot % 64u < 32u && i < {fresh * dim}u) {{"):
-                            i = Aff.of(Atom("i", fresh * dim - 1))
-                            row, column = k.div(i, dim), k.mod(i, dim)
+                    # The first and the second halves of the rows (the two sides of a rotary embedding) on waves of their
+                    # own, so that no wave diverges; in the one-wave-per-head kernel on the waves that stage no q.
+                    half = max(1, dim // 2) if dim % 2 == 0 else dim
+                    sides, per_side = dim // half, -(-fresh * half // 64) * 64
+                    first = staging_from[0] % threads if threads else 0
+                    staging_from[0] += sides * per_side
+                    thread = f"(threadIdx.x + {threads - first}u) % {threads}u" if first else "threadIdx.x"
+                    with k.block(f"for (uint32_t slot = {thread}; slot < {sides * per_side}u; slot += blockDim.x) {{"):
+                        k.line(f"const uint32_t rest = slot % {per_side}u;")
+                        with k.block(f"if (rest < {fresh * half}u) {{"):
+                            rest = Aff.of(Atom("rest", fresh * half - 1))
+                            row, within = k.div(rest, half), k.mod(rest, half)
+                            column = within + k.derived(Aff.of(Atom("slot", sides * per_side - 1)), f"({{}}) / {per_side}u * {half}u", dim - half) if sides > 1 else within
                             node = self.read(k, new_value, [row, h, column])
                             k.hoist_loads(node)
-                            k.line(f"{name}_new[i] = {k.emit(node)};")
+                            k.line(f"{name}_new[{(row.scale(dim) + column).code()}] = {k.emit(node)};")
                 if fresh_only is not None:
                     return
 
-            if past_value is None:
+            if past_value is None or past == 0:
                 if staged:
                     with k.block(f"auto {name} = [&](uint32_t j, uint32_t d) -> float {{", "};"):
                         k.line(f"return {name}_new[j * {dim}u + d];")
@@ -2637,10 +2643,13 @@ class HIPCodegen(Codegen):
                 return self.read(k, past_value, [Aff.of(Atom("j", past - 1)), h, c[1]])
 
             if staged:
-                with k.block(f"auto {name} = [&](uint32_t j, uint32_t d) -> float {{", "};"):
-                    with k.block(f"if (j < {past}u) {{"):
-                        k.line(f"return {k.emit(first([Aff.of(Atom('j', keys - 1)), Aff.of(Atom('d', dim - 1))]))};")
-                    k.line(f"return {name}_new[(j - {past}u) * {dim}u + d];")
+                # both sources read at clamped rows: a load behind a branch would end it with a round trip of its own
+                with k.block(f"auto {name} = [&](uint32_t at, uint32_t d) -> float {{", "};"):
+                    k.line(f"const uint32_t j = at < {past}u ? at : {past - 1}u;")
+                    node = first([Aff.of(Atom('j', past - 1)), Aff.of(Atom('d', dim - 1))])
+                    k.line(f"const float old = {k.emit(node)};")
+                    k.line(f"const float fresh = {name}_new[(at < {past}u ? 0u : at - {past}u) * {dim}u + d];")
+                    k.line(f"return at < {past}u ? old : fresh;")
                 return
 
             def second(c):

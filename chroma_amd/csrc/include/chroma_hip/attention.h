@@ -264,8 +264,16 @@ __device__ __forceinline__ void attention_waves(uint32_t keys, float scale, Load
     __shared__ float q_s[G][D];
     const uint32_t tid = threadIdx.x, lane = tid % kWave, g = tid / kWave;
     const float neg_inf = -__builtin_inff();
-    for (uint32_t i = tid; i < uint32_t(G * D); i += blockDim.x) {
-        q_s[i / D][i % D] = load_q(i / D, i % D);
+    if constexpr (D % 2 == 0) {
+        // the two halves of the rows apart: with whole waves on either, a rotary embedding's branch does not diverge
+        for (uint32_t i = tid; i < uint32_t(G * D); i += blockDim.x) {
+            const uint32_t rest = i % uint32_t(G * D / 2), row = rest / (D / 2), d = i / uint32_t(G * D / 2) * (D / 2) + rest % (D / 2);
+            q_s[row][d] = load_q(row, d);
+        }
+    } else {
+        for (uint32_t i = tid; i < uint32_t(G * D); i += blockDim.x) {
+            q_s[i / D][i % D] = load_q(i / D, i % D);
+        }
     }
     __syncthreads();
     float q[D];
@@ -286,6 +294,96 @@ __device__ __forceinline__ void attention_waves(uint32_t keys, float scale, Load
     // Each lane takes keys lane, lane + 64, ... in that order; U of them per batch, their loads issued
     // together (a batch's keys past the end read the last key and contribute nothing).
     constexpr int U = D <= 16 ? 8 : (D <= 32 ? 4 : 2);
+    if constexpr (D <= kWave && (D & (D - 1)) == 0) {
+        if (keys <= uint32_t(U) * kWave) {  // (``keys`` is a literal: the branch and the unused batches fold away)
+            // One batch: every key's row is requested before any arithmetic, the value rows behind them while both fit
+            // the registers (else once the scores are done), and each score is computed once.
+            const bool together = (keys + kWave - 1u) / kWave * D <= 80u;
+            float k[U][D], v[U][D], m[U], p[U];
+            auto each = [&](auto&& body) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (u * kWave < keys) {
+                        const uint32_t j = lane + u * kWave;
+                        body(u, j < keys ? j : keys - 1u);
+                    }
+                }
+            };
+            auto values = [&](int u, uint32_t j) {
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    v[u][d] = load_v(j, d);
+                }
+            };
+            each([&](int u, uint32_t j) {
+                m[u] = load_mask(j, g);
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    k[u][d] = load_k(j, d);
+                }
+            });
+            if (together) {
+                each(values);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            float peak = load_sink(g);
+            const float sink = peak;
+            each([&](int u, uint32_t) {
+                float dot = 0.0f;
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    dot += q[d] * k[u][d];
+                }
+                const float s = storage_round<BF16>(dot);
+                const float s1 = storage_round<BF16>(s * scale);
+                p[u] = storage_round<BF16>(s1 + m[u]);
+                peak = __builtin_fmaxf(peak, lane + u * kWave < keys ? p[u] : neg_inf);
+            });
+            if (!together) {
+                each(values);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            peak = wave_max(peak);
+            float total = 0.0f;
+            each([&](int u, uint32_t) {
+                p[u] = lane + u * kWave < keys ? fast_exp(p[u] - peak) : 0.0f;
+                total += p[u];
+            });
+            total = wave_sum(total) + fast_exp(sink - peak);
+            float acc[D];
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                acc[d] = 0.0f;
+            }
+            each([&](int u, uint32_t) {
+                const float weight = storage_round<BF16>(p[u] / total);
+                const bool live = lane + u * kWave < keys;  // (a key past the end adds nothing, also where the last value row is infinite)
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    acc[d] += live ? weight * v[u][d] : 0.0f;
+                }
+            });
+            // the lanes' sums, halving the dimensions a lane keeps at every step: lane l ends with dimension l / (64 / D)
+#pragma unroll
+            for (int half = D / 2, offset = kWave / 2; half > 0; half /= 2, offset /= 2) {
+                const bool upper = (lane & uint32_t(offset)) != 0;
+#pragma unroll
+                for (int d = 0; d < half; ++d) {
+                    const float other = __shfl_xor(upper ? acc[d] : acc[d + half], offset, kWave);
+                    acc[d] = (upper ? acc[d + half] : acc[d]) + other;
+                }
+            }
+            float sum = acc[0];
+#pragma unroll
+            for (int offset = kWave / D / 2; offset > 0; offset /= 2) {
+                sum += __shfl_xor(sum, offset, kWave);
+            }
+            if (lane % (kWave / D) == 0) {
+                store(g, lane / (kWave / D), sum);
+            }
+            return;
+        }
+    }
     float peak = neg_inf, total = 0.0f;
     for (uint32_t j0 = lane; j0 < keys; j0 += U * kWave) {
         float s[U];
