@@ -124,10 +124,13 @@ TILED_LOAD_GBS = {(256, 192): 36.0, (128, 192): 44.0}
 # rounds of the chip's 256, now with longer tiles among them), on 192 x 4 waves with 160 236 us, but 276 us
 # against 241 us on the skewed routing the seeded C5 model produces (expert counts 0-1842 at layer 19).
 RING_EXPERT_TILES = ((384, 8, 160), (320, 4, 128))
-# With up to FEW_EXPERT_SLOTS slots an expert (mostly one row tile each, a stream over the weights) a product that would take
-# the 320-channel tile takes this one where its channels allow: 2880 channels of 32 experts are then 480 tiles, two nearly
-# full rounds of the chip, instead of 288, one and an eighth (GPT-OSS-20B's layer of 100 tokens 350 -> 324 us, of 400
-# 414 -> 394; at 800 tokens, 100 slots an expert, 499 and 498; 240-, 480- and 160-channel tiles are slower at 100).
+# With up to FEW_EXPERT_SLOTS slots an expert (mostly one row tile each, a stream over the weights) a product takes
+# FEW_SLOT_TILE instead where its channels allow and the rounds of the chip that the tiles of the experts in use need come
+# out shorter (``_ring_tile``). 2880 channels of 32 experts are then 480 tiles, two nearly full rounds, instead of 288 of 320
+# channels, one and an eighth (GPT-OSS-20B's layer of 100 tokens 350 -> 324 us, of 400 414 -> 394; at 800 tokens, 100 slots
+# an expert, 499 and 498), and 5760 channels of the 25 experts that 12 tokens use 750 tiles, three rounds, instead of 375 of
+# 384 channels, two rounds twice as long (layer of 8 tokens 246 -> 229 us, of 12 277 -> 265; 50 tokens, four rounds of either
+# length in sum, 313 and 316). 240-, 480- and 160-channel tiles are slower at 100 tokens.
 FEW_EXPERT_SLOTS = 64
 FEW_SLOT_TILE = (192, 4, 128)
 # A gated activation between two expert products is computed in the first product's epilogue (no map
@@ -147,6 +150,10 @@ SMALL_REDUCTION = 8  # contractions summing at most this many products are fused
 SMALL_OPERAND_COST = 8  # ...over operands that cost at most this much per element (others are stored)
 MATRIX_MIN_WORK = 1 << 18  # smaller batched products stay on the generic contraction kernel
 GROUPED_SLOTS = 64  # from this many (token, expert) slots on, expert products are grouped by expert
+# ...and from one slot per expert on, bfloat16 products on a ring tile whose slabs would be streamed again for the slots that
+# share an expert, this many bytes or more in sum (12 us of the weight stream, what the routing costs). GPT-OSS-20B's layer:
+# 6 tokens 208 us by slots and 231 by experts, 8 tokens 264 and 229, 10 tokens 324 and 256, 15 tokens 482 and 291.
+REPEATED_SLAB_BYTES = 64 << 20
 FUSED_ROUTER_BYTES = 32 << 10  # a router with gate weights up to this size is recomputed inside its first expert product
 EARLY_FETCH_BYTES = 1 << 20  # weight streams up to this size are requested before their staging prologue
 ROUTER_TICKETS = 48  # rows a split router can serve (chroma::kRouterTickets words of the error region)
@@ -2952,7 +2959,8 @@ class HIPCodegen(Codegen):
         per_slot = eqn == "beck,bek->bec"
         per_expert = "true" if per_slot else "false"
         plan = self._stream_plan(1, inner, out.dtype, tokens * selected * channels * inner * ITEMSIZE[out.dtype])
-        if (tokens * selected < GROUPED_SLOTS and plan is not None and inner <= STAGED_FLOATS
+        grouped = tokens * selected >= GROUPED_SLOTS or self._repeated_slabs(weight, x, tokens * selected, experts, channels, inner)
+        if (not grouped and plan is not None and inner <= STAGED_FLOATS
                 and weight.view.offset % (16 // ITEMSIZE[weight.dtype]) == 0):
             # One slot per workgroup row of the grid: the slot's input row (per token or per slot; any
             # view or fused expression, e.g. the gated activation of the first expert product) is
@@ -2997,7 +3005,7 @@ class HIPCodegen(Codegen):
         if per_slot and not x.stored:
             x = self._activation_epilogue(x) or x
         x = self.contiguous(x)
-        if tokens * selected >= GROUPED_SLOTS and inner % (8 if meta.dtype == torch.bfloat16 else 4) == 0 and experts <= 4096:
+        if grouped and inner % (8 if meta.dtype == torch.bfloat16 else 4) == 0 and experts <= 4096:
             self._grouped_experts(out, weight, indices, x, tokens, selected, experts, channels, inner, per_slot)
             self.expert_contractions += 1
             return out
@@ -3166,9 +3174,7 @@ class HIPCodegen(Codegen):
         split = self._kwave_experts(weight, x, tokens * selected, experts, channels, inner)
         if split is not None:
             return self._kwave_grouped_kernel(out, weight, indices, x, tokens, selected, experts, channels, inner, per_slot, split, activation, store_product)
-        ring = next(((n, w, t) for n, w, t in RING_EXPERT_TILES if channels % n == 0), None)
-        if ring is not None and ring[0] == 320 and channels % FEW_SLOT_TILE[0] == 0 and tokens * selected <= FEW_EXPERT_SLOTS * experts:
-            ring = FEW_SLOT_TILE
+        ring = self._ring_tile(tokens * selected, experts, channels)
         if out.dtype == torch.bfloat16 and inner % 32 == 0 and ring is not None:
             path, (width, waves, last) = 3, ring
             threads = 64 * waves
@@ -3194,6 +3200,30 @@ class HIPCodegen(Codegen):
             f"{inner}u{epilogue});"
         )
         return k, 8 * -(-(-(-channels // width) * tiles) // 8), threads, path, scratch
+
+    @staticmethod
+    def _used_experts(slots: int, experts: int) -> float:
+        """The experts that this many evenly drawn slots meet."""
+        return experts * (1.0 - (1.0 - 1.0 / experts) ** slots)
+
+    @classmethod
+    def _ring_tile(cls, slots: int, experts: int, channels: int) -> Optional[Tuple[int, int, int]]:
+        """The ring body's (channels, waves, slots of a last tile) for a grouped product, or None."""
+        ring = next((tile for tile in RING_EXPERT_TILES if channels % tile[0] == 0), None)
+        if ring is None or channels % FEW_SLOT_TILE[0] or slots > FEW_EXPERT_SLOTS * experts:
+            return ring
+        used = cls._used_experts(slots, experts)
+        return min((ring, FEW_SLOT_TILE), key=lambda tile: math.ceil(used * (channels // tile[0]) / MFMA_CUS) * tile[0])
+
+    @classmethod
+    def _repeated_slabs(cls, weight: Value, x: Value, slots: int, experts: int, channels: int, inner: int) -> bool:
+        """Whether fewer than GROUPED_SLOTS slots are grouped all the same (see REPEATED_SLAB_BYTES). (Operands that start
+        inside a 16-byte chunk stay where they were.)"""
+        if weight.dtype != torch.bfloat16 or inner % 32 or slots < experts or cls._ring_tile(slots, experts, channels) is None:
+            return False
+        if any(v.view is not None and v.view.offset % 8 for v in (weight, x)):
+            return False
+        return (slots - cls._used_experts(slots, experts)) * channels * inner * ITEMSIZE[weight.dtype] >= REPEATED_SLAB_BYTES
 
     def _kwave_experts(self, weight: Value, x: Value, slots: int, experts: int, channels: int, inner: int) -> Optional[Tuple[int, int]]:
         """(16-slot blocks, 16-channel blocks) of the K-split grouped body's pieces, chosen by ``_kwave_plan``'s account over

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import chroma_amd
+from chroma_amd._src.codegen import hip
 from chroma_amd._src.codegen.hip import HIPCodegen
 from chroma_amd._src.compiler import lower_program
 from tests.helpers import Function, as_float, export
@@ -150,6 +151,80 @@ def test_k_split_expert_products(tmp_path, dtype, experts, channels, inner, coun
     w = weights.double()[indices]
     assert_sums(up, torch.einsum("beck,bk->bec", w, x.double()), inner, 0.05, dtype)
     assert_sums(down, torch.einsum("beck,bek->bec", w, per_slot.double()), inner, 0.05, dtype)
+
+
+def few_slots(experts, channels, inner, slots):
+    generator = torch.Generator().manual_seed(slots + channels)
+    weights = (torch.randn(experts, channels, inner, generator=generator) * 0.05).bfloat16()
+    indices = torch.randint(0, experts, (slots, 1), generator=generator)
+    return weights, indices, torch.randn(slots, inner, generator=generator).bfloat16(), torch.randn(slots, 1, inner, generator=generator).bfloat16()
+
+
+def test_few_slots_are_grouped_where_slabs_repeat(monkeypatch):
+    """From one slot per expert on, and only where the repeated slabs cost more than the routing; an operand that starts
+    inside a 16-byte chunk stays on the stream."""
+    of = lambda slots, *view: plan_of(GroupedExperts(), *few_slots(6, 384, 64, slots))
+    assert "grouped_expert" not in of(12)
+    monkeypatch.setattr(hip, "REPEATED_SLAB_BYTES", 1)
+    assert of(5).count("chroma::stream_expert_linear") == 2 and of(6).count("chroma::grouped_expert_linear<") == 2
+    shifted = lambda w, i, x: torch.einsum("beck,bk->bec", w[4:4 + 6 * 384 * 64].reshape(6, 384, 64)[i], x)
+    plan = plan_of(Function(shifted), torch.ones(6 * 384 * 64 + 8, dtype=torch.bfloat16), *few_slots(6, 384, 64, 12)[1:3])
+    assert "grouped_expert" not in plan
+
+
+def test_ring_tiles_of_few_slots():
+    """The narrower tile only where it needs fewer rounds of the chip, and never above its range."""
+    few, wide = hip.FEW_SLOT_TILE, hip.RING_EXPERT_TILES
+    assert [HIPCodegen._ring_tile(slots, 32, 5760) for slots in (32, 200, 2048, 2049)] == [few, wide[0], wide[0], wide[0]]
+    assert [HIPCodegen._ring_tile(slots, 32, 2880) for slots in (32, 200, 2048, 2049)] == [wide[1], few, few, wide[1]]
+    assert HIPCodegen._ring_tile(64, 32, 192) is None and HIPCodegen._ring_tile(64, 32, 640) == wide[1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("experts, channels, inner, slots", [
+    (5, 384, 64, 5),     # the 192-channel tile in place of the 384-channel one
+    (1, 960, 96, 63),    # one expert; the 192-channel tile in place of the 320-channel one
+    (9, 320, 160, 23),   # the 320-channel tile
+])
+def test_few_slots_grouped_by_expert(tmp_path, monkeypatch, experts, channels, inner, slots):
+    monkeypatch.setattr(hip, "REPEATED_SLAB_BYTES", 0)
+    weights, indices, x, per_slot = few_slots(experts, channels, inner, slots)
+    indices[0, 0] -= experts
+    exported = export(GroupedExperts(), weights, indices, x, per_slot)
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        assert (tmp_path / "hip" / "model.hip").read_text().count("chroma::grouped_expert_linear<") >= 1
+        up, down = model(weights, indices, x, per_slot)
+        indices[-1, -1] = experts
+        with pytest.raises(IndexError):
+            model(weights, indices, x, per_slot)
+        indices[-1, -1] = 0
+    indices = few_slots(experts, channels, inner, slots)[1]
+    w = weights.double()[indices]
+    assert_sums(up, torch.einsum("beck,bk->bec", w, x.double()), inner, 0.05, torch.bfloat16)
+    assert_sums(down, torch.einsum("beck,bek->bec", w, per_slot.double()), inner, 0.05, torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("keys, dim", [
+    (2, 16), (64, 16), (65, 16), (512, 16),   # one past key, whole and ragged rounds of 64 keys, the longest single batch
+    (256, 32), (257, 32), (128, 64), (129, 64),  # value rows requested behind the scores; two batches
+    (70, 8), (70, 24),                        # more lanes to a dimension; no power of two
+])
+def test_one_wave_per_head_attention(tmp_path, dtype, keys, dim):
+    """One query on one wave per head, against the oracle: at its bfloat16 bar, or (float) within the errors of sums of up
+    to 513 terms and of an exponential of arguments up to about 20 (2^-24 times either, and a few such)."""
+    from oracle import compile_cpu
+    from tests.helpers import assert_close, numpy_of
+    from tests.test_hip_runtime import SinkAttention
+
+    inputs = tuple(v.to(dtype) for v in attention_inputs(1, keys - 1, 2, 4, dim, None))
+    exported = torch.export.export(SinkAttention(), inputs)
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        got = [model(*inputs) for _ in range(2)]
+    want = compile_cpu(exported, tmp_path / "cpu")(*[numpy_of(v) for v in inputs])
+    for result in got:
+        assert_close(result, want, **({"rtol": 2e-2, "atol": 1e-2} if dtype == torch.bfloat16 else {"rtol": 1e-4, "atol": 1e-5}))
 
 
 @pytest.mark.gpu
