@@ -17,7 +17,10 @@
 //
 // Rounding: the scores, scaled scores and masked scores are rounded as attention.h says; a probability is rounded to
 // bfloat16 as exp(s - m), m a running maximum of the row, before it meets V, and the row is divided by the float sum at
-// the end (the same relative rounding of each probability as when it is divided first).
+// the end (the same relative rounding of each probability as when it is divided first). Where every wave has at most one
+// block (up to 256 keys, one workgroup a row group) the waves exchange their (max, sum) before the second product and
+// the probabilities are divided first, as attention.h's are: a row of few live keys then has the very probabilities of
+// the unfused chain, at the price of one barrier.
 #pragma once
 
 #include "attention.h"
@@ -64,6 +67,8 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
     const float neg_inf = -__builtin_inff();
     T* ks = lds + wave * WAVE;
     T* vs = ks + kFlashKeys * D;
+    __shared__ float stats[BF16 ? kFlashWaves : 1][BF16 ? ROWS : 1][2];
+    const bool divided = BF16 && splits == 1u && a.keys <= kFlashWaves * kFlashKeys;
 
     uint32_t query[RT];
     uint4 qf[RT][PARTS];
@@ -154,6 +159,15 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
     if (n < mine) {
         copy_k(first + n * stride);
         copy_v(first + n * stride);
+    }
+    if constexpr (BF16) {
+        if (divided && mine == 0u) {  // (a wave without a block; the others meet it at the barrier in the loop, run once)
+            for (uint32_t r = lane; r < ROWS; r += 64u) {
+                stats[wave][r][0] = neg_inf;
+                stats[wave][r][1] = 0.0f;
+            }
+            __syncthreads();
+        }
     }
     while (n < mine) {
         const uint32_t block = first + n * stride, next = next_of(n + 1u);
@@ -248,21 +262,56 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
             const float shift = peak[rt] == neg_inf ? 0.0f : -peak[rt] * kLog2e;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                float e[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    e[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(u[rt][t][r], kLog2e, shift));
-                    total[rt] += e[r];
+                    u[rt][t][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(u[rt][t][r], kLog2e, shift));
+                    total[rt] += u[rt][t][r];
                 }
+            }
+        }
+        if constexpr (BF16) {
+            float factor[RT];
 #pragma unroll
-                for (int r = 0; r < 4; r += 2) {
-                    if constexpr (BF16) {
-                        const bf16x2_t pair = __builtin_convertvector(f32x2_t{e[r], e[r + 1]}, bf16x2_t);
+            for (int rt = 0; rt < RT; ++rt) {
+                factor[rt] = 1.0f;
+            }
+            if (divided) {
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    float sum = total[rt] + __shfl_xor(total[rt], 16, kWave);
+                    sum += __shfl_xor(sum, 32, kWave);
+                    if (quad == 0) {
+                        stats[wave][rt * 16 + col][0] = peak[rt];
+                        stats[wave][rt * 16 + col][1] = sum;
+                    }
+                }
+                __syncthreads();
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const uint32_t row = row0 + rt * 16u + col < total_rows ? row0 + rt * 16u + col : total_rows - 1u;
+                    const float sink = widen_of<T>(a.sinks[kv * a.sh + (row % G) * a.sg]);
+                    FlashMerge merge{sink, 0.0f};
+#pragma unroll
+                    for (uint32_t w = 0; w < kFlashWaves; ++w) {
+                        merge.top = __builtin_fmaxf(merge.top, stats[w][rt * 16 + col][0]);
+                    }
+#pragma unroll
+                    for (uint32_t w = 0; w < kFlashWaves; ++w) {
+                        merge.total += merge.weight(stats[w][rt * 16 + col][0]) * stats[w][rt * 16 + col][1];
+                    }
+                    merge.total += merge.weight(sink);
+                    factor[rt] = merge.weight(peak[rt]) / merge.total;
+                }
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                    for (int r = 0; r < 4; r += 2) {
+                        const bf16x2_t pair = __builtin_convertvector(f32x2_t{u[rt][t][r] * factor[rt], u[rt][t][r + 1] * factor[rt]}, bf16x2_t);
                         pf[rt][t / 2][t % 2 * 4 + r] = pair[0];
                         pf[rt][t / 2][t % 2 * 4 + r + 1] = pair[1];
-                    } else {
-                        u[rt][t][r] = e[r];
-                        u[rt][t][r + 1] = e[r + 1];
                     }
                 }
             }
@@ -351,13 +400,13 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
         f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (uint32_t w = 0; w < kFlashWaves; ++w) {
-            const float scale = merge.weight(parts[w * PART + ROWS * OPAD + 2u * r]);
+            const float scale = divided ? 1.0f : merge.weight(parts[w * PART + ROWS * OPAD + 2u * r]);
             merge.total += scale * parts[w * PART + ROWS * OPAD + 2u * r + 1u];
             sum += scale * *reinterpret_cast<const f32x4_t*>(parts + w * PART + r * OPAD + d);
         }
         if (splits == 1u) {
             merge.total += merge.weight(sink);
-            sum *= 1.0f / merge.total;
+            sum *= divided ? 1.0f : 1.0f / merge.total;
             const float y[4] = {sum[0], sum[1], sum[2], sum[3]};
             kwave_store<T>(a.out + ((size_t(row / G) * a.kv_heads + kv) * G + row % G) * D + d, y, d, D);
         } else {
