@@ -258,6 +258,9 @@ __device__ __forceinline__ void attention_rows(uint32_t begin, uint32_t end, flo
 // One query row and one key/value head per workgroup with one wave per query head (blockDim.x = 64 G):
 // for short key ranges the wave's lanes split the keys and every reduction is a wave butterfly, so the
 // workgroup synchronizes only once, after the query rows are staged. Same numerics as attention_rows.
+// A chain of memory round trips (q, then the keys) bounds it, not bytes: a range of up to U rounds of 64 keys therefore
+// requests all of its rows at once. One float query over 257 keys of 16 dimensions, 8 heads, with its output product:
+// 9.9 us when every score was computed twice behind a branch per key, 7.8 us so (one decode step 387 -> 357 us).
 template <int D, int G, bool BF16, class LoadQ, class LoadK, class LoadV, class LoadMask, class LoadSink, class Store>
 __device__ __forceinline__ void attention_waves(uint32_t keys, float scale, LoadQ load_q, LoadK load_k, LoadV load_v, LoadMask load_mask,
                                                 LoadSink load_sink, Store store) {
