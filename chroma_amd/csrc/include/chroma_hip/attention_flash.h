@@ -58,7 +58,6 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
     constexpr int COPIES = kFlashKeys * D * sizeof(T) / 1024;  // 1 KB copies per block and operand
     constexpr int PARTS = PER_ROW / 4u;                        // matrix-core operands of a row: 64 bytes of it each
     constexpr uint32_t SWZ = PER_ROW % 8u == 0 ? 7u : 3u;  // chunk c of row r lies at c ^ ((r / 2) & SWZ)
-    constexpr float kLog2e = 1.44269504088896341f;
     __shared__ __attribute__((aligned(1024))) T lds[kFlashWaves * WAVE];
     const uint32_t lane = threadIdx.x % 64u, quad = lane / 16u, col = lane % 16u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64u);
@@ -259,12 +258,14 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
                 }
                 peak[rt] = top;
             }
-            const float shift = peak[rt] == neg_inf ? 0.0f : -peak[rt] * kLog2e;
+            // subtracted before it is scaled: the rounding of peak * log2(e) alone would grow with the scores (2.6e-6 of a
+            // float result at scores around 100, and an infinite power for a row that has met only a finite masking value)
+            const float base = peak[rt] == neg_inf ? 0.0f : peak[rt];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    u[rt][t][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(u[rt][t][r], kLog2e, shift));
+                    u[rt][t][r] = fast_exp(u[rt][t][r] - base);
                     total[rt] += u[rt][t][r];
                 }
             }
