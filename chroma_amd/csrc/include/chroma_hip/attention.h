@@ -1114,7 +1114,7 @@ template <int D> __device__ __forceinline__ void attention_mfma_bf16(const Atten
 // S^T = K . Q^T on v_mfma_f32_16x16x32_bf16, each score rounded to bfloat16, scaled and rounded, masked
 // and rounded (gfx950's v_cvt_pk_bf16_f32 rounds two values at once, to nearest even like f32_to_bf16);
 // pass 1 accumulates (max, sum of exp) per query in float, pass 2 forms p = exp(s - max) / sum as
-// 2^(s log2(e) - max log2(e) - log2(sum)) - one multiply-add and one v_exp_f32, within a few float ulps
+// 2^((s - max) log2(e) - log2(sum)) - two multiply-adds and one v_exp_f32, within a few float ulps
 // of the quotient, far below the bfloat16 rounding p then gets - and O^T += V^T . P^T; the output is
 // rounded once.
 // The 64-key blocks a query tile visits come from ``attention_live_tiles`` (blocks whose mask is -inf
@@ -1448,14 +1448,15 @@ template <int D, int G, bool POW2, int HPW = 1> __device__ __forceinline__ void 
             }
             top = __builtin_fmaxf(peak[hd], top * cs);  // exact: cs is 1 or a power of two
             if (top != neg_inf) {
-                // exp(s - top) = 2^(u * cs * log2(e) - top * log2(e)): one multiply-add per score
-                const float scale2 = cs * kLog2e, shift = -top * kLog2e;
+                // s - top first, exactly: one multiply-add by log2(e) with top * log2(e) rounded on its own gave infinite
+                // powers where a row had met only a large finite masking value. (The layer of 2048 tokens 319 -> 323 us;
+                // 325 with that multiply-add kept for waves whose maxima are small, behind a branch.)
                 float sum = 0.0f;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        sum += __builtin_amdgcn_exp2f(__builtin_fmaf(u[hd][t][r], scale2, shift));
+                        sum += fast_exp(__builtin_fmaf(u[hd][t][r], cs, -top));
                     }
                 }
                 total[hd] = total[hd] * fast_exp(peak[hd] - top) + sum;
@@ -1464,8 +1465,8 @@ template <int D, int G, bool POW2, int HPW = 1> __device__ __forceinline__ void 
         }
     });
     // Combine the four lane groups that share a query, then fold in the sink.
-    // p = exp(s - peak) / total = 2^(s * log2(e) - (peak * log2(e) + log2(total))): the normalisation
-    // rides in the exponent's one multiply-add (v_log_f32 is log2). Only a row whose scores and sink are
+    // p = exp(s - peak) / total = 2^((s - peak) * log2(e) - log2(total)): the normalisation rides in the
+    // exponent's second multiply-add (v_log_f32 is log2). Only a row whose scores and sink are
     // all -inf has total 0; its probabilities are NaN, as the reference's 0 / 0 is.
     float norm[HPW];
 #pragma unroll
@@ -1475,7 +1476,7 @@ template <int D, int G, bool POW2, int HPW = 1> __device__ __forceinline__ void 
             softmax_stats_merge(peak[hd], total[hd], __shfl_xor(peak[hd], offset, kWave), __shfl_xor(total[hd], offset, kWave));
         }
         softmax_stats_add(peak[hd], total[hd], bf16_to_f32(a.sinks[kv * a.sh + (g0 + hd) * a.sg]));
-        norm[hd] = -(peak[hd] * kLog2e + __builtin_amdgcn_logf(total[hd]));
+        norm[hd] = -__builtin_amdgcn_logf(total[hd]);
     }
 
     f32x4_t o[HPW][D / 16];
@@ -1488,7 +1489,7 @@ template <int D, int G, bool POW2, int HPW = 1> __device__ __forceinline__ void 
     }
     sweep(true, [&](int buffer, uint32_t entry) {
         float u[HPW][4][4];
-        const float scale2 = scores(buffer, entry, u) * kLog2e;
+        const float cs = scores(buffer, entry, u);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             // keys 32 h + (4 quad + r) and 32 h + 16 + (4 quad + r): this lane's B operand slots 0-3 and 4-7
@@ -1498,7 +1499,7 @@ template <int D, int G, bool POW2, int HPW = 1> __device__ __forceinline__ void 
                 float e[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(u[hd][2 * h + i / 4][i % 4], scale2, norm[hd]));
+                    e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(__builtin_fmaf(u[hd][2 * h + i / 4][i % 4], cs, -peak[hd]), kLog2e, norm[hd]));
                 }
 #pragma unroll
                 for (int i = 0; i < 8; i += 2) {

@@ -90,16 +90,23 @@ FLASH = [  # tokens, past, KV heads, group, dim, window
     (BF16, 70, 900, 1, 8, 128, 500),
 ]
 
+HEADS = [  # the group-shared prefill kernel: two heads a wave, one; a power-of-two scale, another
+    (BF16, 100, 200, 2, 4, 64, 90),
+    (BF16, 130, 101, 1, 3, 64, 70),
+    (BF16, 70, 140, 2, 2, 128, 100),
+]
+
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype, tokens, past, kv_heads, group, dim, window", FLASH)
-def test_few_query_attention_with_finite_masks(tmp_path, dtype, tokens, past, kv_heads, group, dim, window):
+@pytest.mark.parametrize("kernel, dtype, tokens, past, kv_heads, group, dim, window",
+                         [("attention_flash<", *case) for case in FLASH] + [("attention_heads_mfma_bf16<", *case) for case in HEADS])
+def test_attention_with_finite_masks(tmp_path, kernel, dtype, tokens, past, kv_heads, group, dim, window):
     """Masked keys filled with -inf and with finite values down to the type's lowest: rows that see no key in whole key
     blocks, and a row that sees none at all."""
     q, k, v, sinks, seen = operands(tokens, past, kv_heads, group, dim, dtype, window)
     model, call, source = compiled(tmp_path, dtype, tokens, past, kv_heads, group, dim)
     with model:
-        assert "attention_flash<" in source
+        assert kernel in source
         for fill in (-math.inf, -3e4, -1e10, -1e30, torch.finfo(dtype).min):
             mask = torch.where(seen, 0.0, torch.tensor(fill)).to(dtype)
             assert_attention(call(q, k, v, mask, sinks), q, k, v, mask, sinks)
