@@ -194,6 +194,13 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));  // K, V and the mask of this block
         __builtin_amdgcn_sched_barrier(0);
+        if (block * kFlashKeys + kFlashKeys > a.keys) {
+            // the copies of the last key stand for none: their probability is 0, and 0 times an infinite value would be NaN
+            const uint32_t from = (a.keys - block * kFlashKeys) * PER_ROW;
+            for (uint32_t c = from + lane; c < kFlashKeys * PER_ROW; c += 64u) {
+                *reinterpret_cast<uint4*>(vs + c * CHUNK) = uint4{0u, 0u, 0u, 0u};
+            }
+        }
         // scores of keys 16 t + 4 quad + r for this lane's row, in u units: s = u * cs (attention_heads_mfma_bf16)
         float u[RT][4][4];
 #pragma unroll

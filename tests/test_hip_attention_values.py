@@ -132,3 +132,22 @@ def test_float_attention_with_large_scores(tmp_path, tokens, past, kv_heads, gro
             error = np.linalg.norm((got - want)[live]) / np.linalg.norm(want[live])
             print(f"scores around {base}: {error:.2e}", flush=True)
             assert error < 8 * 2.0**-24, (base, error)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype, tokens, past, kv_heads, group, dim", [
+    (F32, 20, 100, 2, 3, 32), (F32, 130, 1103, 1, 8, 64),                        # one split, three
+    (BF16, 5, 150, 2, 3, 32), (BF16, 40, 301, 8, 16, 64), (BF16, 33, 700, 1, 1, 64),  # divided first, in the end, split
+])
+def test_infinite_last_value_row(tmp_path, dtype, tokens, past, kv_heads, group, dim):
+    """The last key block is ragged and the last key's values are infinite: every query sees that key, so every result is
+    infinite, and nothing of the block behind it turns it into NaN."""
+    q, k, v, sinks, seen = operands(tokens, past, kv_heads, group, dim, dtype, 10**6)
+    assert len(k) % 64
+    v[-1, :, ::2], v[-1, :, 1::2] = math.inf, -math.inf
+    mask = torch.zeros(seen.shape, dtype=dtype)
+    model, call, source = compiled(tmp_path, dtype, tokens, past, kv_heads, group, dim)
+    with model:
+        assert "attention_flash<" in source
+        got = as_float(call(q, k, v, mask, sinks))
+    assert (got[..., ::2] == math.inf).all() and (got[..., 1::2] == -math.inf).all(), np.isnan(got).sum()
