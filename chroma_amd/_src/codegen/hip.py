@@ -2258,7 +2258,8 @@ class HIPCodegen(Codegen):
         args = [self._matrix_slot(k, x), self._matrix_slot(k, weight), self._matrix_slot(k, bias) if bias is not None else "nullptr"]
         out_slot = k.slot(out.name, out.dtype, writable=True, extent=self.extents[out.name])
         slots = min(4, KWAVE_LDS // (KWAVE_WAVES * (tm + tn) << 10))
-        k.line(f"chroma::kwave_linear<{ctype_of(out.dtype)}, {tm}, {tn}, {KWAVE_WAVES}, {slots}>({args[0]}, {args[1]}, {args[2]}, {out_slot}, "
+        fine = str(rows <= 16 and out.dtype == torch.float32).lower()  # (the rows of the weight stream, whose sums are as short)
+        k.line(f"chroma::kwave_linear<{ctype_of(out.dtype)}, {tm}, {tn}, {KWAVE_WAVES}, {slots}, {fine}>({args[0]}, {args[1]}, {args[2]}, {out_slot}, "
                f"{rows}u, {columns}u, {inner}u);")
         tiles = -(-rows // (16 * tm)) * -(-columns // (16 * tn))
         self.launch(k, 8 * -(-tiles // 8), 64 * KWAVE_WAVES, [x, weight] + ([bias] if bias is not None else []), kind="linear_kwave")

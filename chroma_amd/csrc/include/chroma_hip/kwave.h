@@ -30,7 +30,15 @@ __device__ __forceinline__ void kwave_mfma(const uint4& b, const uint4& a, f32x4
     }
 }
 
-constexpr uint32_t kKwaveFlush = 4;
+// A float unit's 16 products of one element, summed 8 + 8.
+__device__ __forceinline__ f32x4_t kwave_unit(const uint4& b, const uint4& a) {
+    const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4_t lo = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b.x), __uint_as_float(a.x), zero, 0, 0, 0);
+    f32x4_t hi = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b.z), __uint_as_float(a.z), zero, 0, 0, 0);
+    lo = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b.y), __uint_as_float(a.y), lo, 0, 0, 0);
+    hi = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b.w), __uint_as_float(a.w), hi, 0, 0, 0);
+    return lo + hi;
+}
 
 // Elements of the LDS array: S units of TM + TN 16-row blocks (1 KiB each) per wave; a wave's partial sums (TM TN
 // KiB) take the place of its own ring.
@@ -47,7 +55,7 @@ __device__ __forceinline__ uint32_t kwave_row() { return threadIdx.x % 64u / 4u;
 // 32-bit, so the caller guarantees operands below 2 GiB. ``row_bytes`` (a multiple of 16) is K's extent. The ring's
 // 16-byte chunks are swizzled as the ring body's (``wide_swizzle``). ``store(i, j, v)`` is called once per 16 x 16
 // block (i, j) on the wave that sums it: lane l has row 16 i + l % 16, columns 16 j + 4 (l / 16) .. + 3.
-template <class T, int TM, int TN, int NW, int S, class Store>
+template <class T, int TM, int TN, int NW, int S, bool FINE, class Store>
 __device__ __forceinline__ void kwave_tile(const char* __restrict__ a, const uint32_t (&oa)[TM], const char* __restrict__ b,
                                            const uint32_t (&ob)[TN], uint32_t row_bytes, uint16_t* lds, Store store) {
     static_assert(S >= 2, "a unit being read and at least one in flight");
@@ -60,6 +68,13 @@ __device__ __forceinline__ void kwave_tile(const char* __restrict__ a, const uin
     const uint32_t chunk = 16u * ((lane % 4u) ^ wide_swizzle(lane / 4u));                               // copied byte of the row's unit
     const uint32_t at = (lane % 16u) * 32u + (((lane / 16u) ^ wide_swizzle(lane % 16u)) * 8u);  // fragment element in a block
     const uint32_t tail = row_bytes % 64u;  // bytes of a ragged last unit
+    // Float sums are kept in levels, so that their rounding errors grow with the root of a level's length and not of the whole
+    // (3 x 2880 x 11520: 6.2e-7 relative in one chain, 1.9e-7 with levels of FLUSH = 4 units, a wave's share, the waves).
+    // FINE adds a unit's two halves of 8 products and takes 8 units a level, as exact as the weight stream it stands in for:
+    // 8 x 4096 x 1024 9.6e-8 (1.55e-7 without), 3 x 2880 x 11520 1.3e-7. Its additions cost nothing beside the copies of few
+    // rows, but a product of many rows is bound by the matrix cores: 1000 rows, 1024 -> 4096, +16%.
+    constexpr bool LEVELS = sizeof(T) == 4;
+    constexpr uint32_t FLUSH = FINE ? 8u : 4u;
     f32x4_t acc[TM][TN];
     unroll<TM>([&](auto i) { unroll<TN>([&](auto j) { acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}; }); });
     // past the row's end (a ragged last unit) a lane copies the unit's first 16 bytes instead; the reader drops them
@@ -86,23 +101,28 @@ __device__ __forceinline__ void kwave_tile(const char* __restrict__ a, const uin
             unroll<TM>([&](auto i) { fa[i] = uint4{0u, 0u, 0u, 0u}; });
             unroll<TN>([&](auto j) { fb[j] = uint4{0u, 0u, 0u, 0u}; });
         }
-        unroll<TM>([&](auto i) { unroll<TN>([&](auto j) { kwave_mfma<T>(fb[j], fa[i], acc[i][j]); }); });
+        unroll<TM>([&](auto i) {
+            unroll<TN>([&](auto j) {
+                if constexpr (LEVELS && FINE) {
+                    acc[i][j] += kwave_unit(fb[j], fa[i]);
+                } else {
+                    kwave_mfma<T>(fb[j], fa[i], acc[i][j]);
+                }
+            });
+        });
     };
     unroll<S - 1>([&](auto n) {
         if (begin + uint32_t(n) < end) {
             copy(begin + uint32_t(n));
         }
     });
-    // Float sums of long rows are kept in two levels, kKwaveFlush units at a time, so their rounding errors grow with the
-    // root of a level's length and not of the whole (3 x 2880 x 11520: 6.2e-7 relative in one level).
-    constexpr bool LEVELS = sizeof(T) == 4;
     f32x4_t sums[LEVELS ? TM : 1][LEVELS ? TN : 1];
     if constexpr (LEVELS) {
         unroll<TM>([&](auto i) { unroll<TN>([&](auto j) { sums[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}; }); });
     }
     auto level = [&](uint32_t u) {
         if constexpr (LEVELS) {
-            if ((u - begin) % kKwaveFlush == kKwaveFlush - 1u || u + 1u == end) {
+            if ((u - begin) % FLUSH == FLUSH - 1u || u + 1u == end) {
                 unroll<TM>([&](auto i) {
                     unroll<TN>([&](auto j) {
                         sums[i][j] += acc[i][j];
@@ -176,7 +196,7 @@ __device__ __forceinline__ void kwave_store(T* to, const float (&y)[4], uint32_t
 // bfloat16 or 4 float values), and X and a column tile of W below 2 GiB. Measured on cold weights, NW = 4, against
 // the 128 x 128 bodies: bfloat16 100 x 5120 x 2880 51.6 -> 18.5 us, 300 x 1024 x 4096 58.9 -> 16.0, 600 x 2880 x 4096
 // 57.3 (the 128 x 192 ring body) -> 32.9; float 256 x 160 x 128 14.3 -> 2.2, 100 x 4000 x 1000 84 -> 15.
-template <class T, int TM, int TN, int NW, int S>
+template <class T, int TM, int TN, int NW, int S, bool FINE>
 __device__ __forceinline__ void kwave_linear(const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias, T* __restrict__ out,
                                              uint32_t m_total, uint32_t n_total, uint32_t k_total) {
     __shared__ __attribute__((aligned(1024))) uint16_t lds[kwave_elements<TM, TN, NW, S>()];
@@ -196,7 +216,7 @@ __device__ __forceinline__ void kwave_linear(const T* __restrict__ x, const T* _
         const uint32_t n = n0 + j * 16u + kwave_row();
         ob[j] = ((n < n_total ? n : n_total - 1u) - n0) * row_bytes;
     });
-    kwave_tile<T, TM, TN, NW, S>(reinterpret_cast<const char*>(x), oa, reinterpret_cast<const char*>(w) + size_t(n0) * row_bytes, ob, row_bytes, lds,
+    kwave_tile<T, TM, TN, NW, S, FINE>(reinterpret_cast<const char*>(x), oa, reinterpret_cast<const char*>(w) + size_t(n0) * row_bytes, ob, row_bytes, lds,
                                  [&](uint32_t i, uint32_t j, f32x4_t v) {
         const uint32_t m = m0 + i * 16u + lane % 16u, n = n0 + j * 16u + 4u * (lane / 16u);
         if (m >= m_total || n >= n_total) {
@@ -292,7 +312,7 @@ __device__ __forceinline__ void grouped_expert_kwave(const T* __restrict__ w, co
             const uint32_t slot = uint32_t(slot_of[r < rows ? r : rows - 1u]);
             oa[i] = (PER_SLOT ? slot : slot / selected) * row_bytes;
         });
-        kwave_tile<T, L, TN, NW, S>(reinterpret_cast<const char*>(x), oa,
+        kwave_tile<T, L, TN, NW, S, false>(reinterpret_cast<const char*>(x), oa,
                                     reinterpret_cast<const char*>(w) + (size_t(expert) * channels + n0) * row_bytes, ob, row_bytes, lds,
                                     [&](uint32_t i, uint32_t j, f32x4_t v) {
             const uint32_t r = i * 16u + lane % 16u, n = n0 + j * 16u + 4u * (lane / 16u);

@@ -68,6 +68,29 @@ def test_k_split_linear(tmp_path, dtype, rows, inner, columns):
         assert_sums(result, exact, inner, 0.05, dtype)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows, inner, columns, levels", [
+    (8, 1024, 4096, (8, 2, 8, 2, 4)),     # products, halves of a unit, units, levels of a wave's share of K, waves
+    (3, 11520, 2880, (8, 2, 8, 22.5, 4)),
+    (40, 4096, 1024, (64, 16, 4)),        # more than 16 rows: levels of 4 units in one chain
+])
+def test_k_split_float_sums(tmp_path, rows, inner, columns, levels):
+    """The rounding errors of float sums in levels. A level of n terms of like size rounds n partial sums whose mean square is
+    (n + 1) / 2 / n of its result's, each by 0.42 x 2^-24 (a uniform error of at most half a spacing, over the spacings of
+    its values), and the squares of the levels add up; a fifth more is allowed (the variance of a sample, sums of
+    unlike size). The weight stream's sums of few rows are as exact: chains of K / 64 products and a tree."""
+    layer, x = linear(rows, inner, columns, torch.float32, bias=False)
+    exported = torch.export.export(layer, (x,))
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        assert "kwave_linear" in (tmp_path / "hip" / "model.hip").read_text()
+        got = model(x)
+    exact = (x.double() @ layer.weight.detach().double().T).numpy()
+    error = np.linalg.norm(got - exact) / np.linalg.norm(exact)
+    limit = 1.2 * 0.42 * 2.0**-24 * sum((n + 1) / 2 for n in levels) ** 0.5
+    print(f"{rows} x {columns} x {inner}: {error:.3e}, limit {limit:.3e}", flush=True)
+    assert error < limit, (error, limit)
+
+
 def attention_inputs(tokens, past, kv_heads, group, dim, window):
     """Operands of a cached attention with sinks: causal (or windowed) over a cache of ``past`` rows, one query row
     wholly masked, an additive bias on a band of keys."""
