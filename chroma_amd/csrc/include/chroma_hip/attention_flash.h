@@ -216,7 +216,11 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
                 const uint4 kf = *reinterpret_cast<const uint4*>(ks + r * D + ((c * 4u + quad) ^ ((r / 2u) & SWZ)) * CHUNK);
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
-                    kwave_mfma<T>(kf, qf[rt][c], s[rt]);
+                    if constexpr (BF16) {
+                        kwave_mfma<T>(kf, qf[rt][c], s[rt]);
+                    } else {
+                        s[rt] += kwave_unit(kf, qf[rt][c]);
+                    }
                 }
             }
 #pragma unroll
@@ -348,9 +352,12 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
             }
         }
         } else {
-            // product (t, r) takes keys 16 t + 4 quad + r: this lane's own probability, V's element (key, d = 16 dt + col)
+            // product (t, r) takes keys 16 t + 4 quad + r: this lane's own probability, V's element (key, d = 16 dt + col).
+            // 16 keys are summed before they join the row's: over 512 keys of 16 the result's error is 1.8e-7 of it
+            // (2.9e-7 with one chain over a wave's keys and over each score's products, 2.1e-7 on the vector units)
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
+                f32x4_t sum[RT][D / 16];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const uint32_t key = t * 16u + quad * 4u + r;
@@ -359,8 +366,16 @@ __device__ __forceinline__ void attention_flash(const AttentionOperandsOf<T>& a,
                         const float v = vs[key * D + ((dt * 4u + col / 4u) ^ ((key / 2u) & SWZ)) * 4u + col % 4u];
 #pragma unroll
                         for (int rt = 0; rt < RT; ++rt) {
-                            o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, u[rt][t][r], o[rt][dt], 0, 0, 0);
+                            const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                            sum[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, u[rt][t][r], r == 0 ? zero : sum[rt][dt], 0, 0, 0);
                         }
+                    }
+                }
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+                    for (int dt = 0; dt < D / 16; ++dt) {
+                        o[rt][dt] += sum[rt][dt];
                     }
                 }
             }

@@ -135,6 +135,28 @@ def test_float_attention_with_large_scores(tmp_path, tokens, past, kv_heads, gro
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tokens, past, kv_heads, group, dim, simulated", [(20, 492, 2, 4, 16, 1.8e-7), (20, 492, 2, 4, 64, 1.8e-7)])
+def test_float_attention_error(tmp_path, tokens, past, kv_heads, group, dim, simulated):
+    """The error of normal operands against 64 bits. The chain simulated in float with the kernel's order of sums (scores in chains of 8
+    products, 16 keys a level, 4 waves) gives ``simulated``, with single chains 2.9e-7 and 3.7e-7, with a thread a key and 32
+    lanes a sum (the vector units' kernel) 2.2e-7 and 3.2e-7; a fifth more is allowed for another sample."""
+    generator = torch.Generator().manual_seed(1)
+    q, k, v, sinks = (torch.randn(shape, generator=generator) * scale for shape, scale in (
+        ((tokens, kv_heads, group, dim), 1.0), ((past + tokens, kv_heads, dim), 1.0), ((past + tokens, kv_heads, dim), 1.0), ((kv_heads * group,), 2.0)))
+    mask = torch.where(torch.arange(past + tokens) <= past + torch.arange(tokens)[:, None], 0.0, -math.inf)
+    model, call, source = compiled(tmp_path, F32, tokens, past, kv_heads, group, dim)
+    with model:
+        assert "attention_flash<" in source
+        got = call(q, k, v, mask, sinks)
+    scores = torch.einsum("qhmd,khd->hmqk", q.double(), k.double()) / math.sqrt(dim) + mask.double()
+    sink = sinks.double().reshape(kv_heads, group, 1, 1).expand(-1, -1, tokens, -1)
+    want = torch.einsum("hmqk,khd->qhmd", torch.softmax(torch.cat((scores, sink), -1), -1)[..., :-1], v.double()).numpy()
+    error = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"head dimension {dim}: {error:.2e}", flush=True)
+    assert error < 1.2 * simulated, (error, simulated)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype, tokens, past, kv_heads, group, dim", [
     (F32, 20, 100, 2, 3, 32), (F32, 130, 1103, 1, 8, 64),                        # one split, three
     (BF16, 5, 150, 2, 3, 32), (BF16, 40, 301, 8, 16, 64), (BF16, 33, 700, 1, 1, 64),  # divided first, in the end, split
