@@ -297,7 +297,9 @@ __device__ __forceinline__ void attention_waves(uint32_t keys, float scale, Load
     // Each lane takes keys lane, lane + 64, ... in that order; U of them per batch, their loads issued
     // together (a batch's keys past the end read the last key and contribute nothing).
     constexpr int U = D <= 16 ? 8 : (D <= 32 ? 4 : 2);
-    if constexpr (D <= kWave && (D & (D - 1)) == 0) {
+    // (More than 8 waves leave a lane 128-168 registers, and rows kept there spill: 288 bytes of scratch a lane at 16 heads of 16
+    // over 320 keys, 360 at 16 of 32 over 256, 544 at 16 of 64 over 100, against 0, 0 and 196 in the batches below.)
+    if constexpr (G <= 8 && D <= kWave && (D & (D - 1)) == 0) {
         if (keys <= uint32_t(U) * kWave) {  // (``keys`` is a literal: the branch and the unused batches fold away)
             // One batch: every key's row is requested before any arithmetic, the value rows behind them while both fit
             // the registers (else once the scores are done), and each score is computed once.

@@ -2,15 +2,20 @@
 
 from __future__ import annotations
 
+import re
+import subprocess
+
 import numpy as np
 import pytest
 import torch
 
 import chroma_amd
+from chroma_amd._src.build import compiler_command
 from chroma_amd._src.codegen import hip
 from chroma_amd._src.codegen.hip import HIPCodegen
 from chroma_amd._src.compiler import lower_program
 from tests.helpers import Function, as_float, export
+from tests.test_hip_runtime import SinkAttention
 
 
 def assert_sums(got, exact, terms, scale, dtype):
@@ -128,7 +133,6 @@ def test_few_query_attention(tmp_path, tokens, past, kv_heads, group, dim, windo
     its bfloat16 bar, twice."""
     from oracle import compile_cpu
     from tests.helpers import assert_close, numpy_of
-    from tests.test_hip_runtime import SinkAttention
 
     inputs = attention_inputs(tokens, past, kv_heads, group, dim, window)
     exported = torch.export.export(SinkAttention(), inputs)
@@ -239,7 +243,6 @@ def test_one_wave_per_head_attention(tmp_path, dtype, keys, dim):
     to 513 terms and of an exponential of arguments up to about 20 (2^-24 times either, and a few such)."""
     from oracle import compile_cpu
     from tests.helpers import assert_close, numpy_of
-    from tests.test_hip_runtime import SinkAttention
 
     inputs = tuple(v.to(dtype) for v in attention_inputs(1, keys - 1, 2, 4, dim, None))
     exported = torch.export.export(SinkAttention(), inputs)
@@ -248,6 +251,41 @@ def test_one_wave_per_head_attention(tmp_path, dtype, keys, dim):
     want = compile_cpu(exported, tmp_path / "cpu")(*[numpy_of(v) for v in inputs])
     for result in got:
         assert_close(result, want, **({"rtol": 2e-2, "atol": 1e-2} if dtype == torch.bfloat16 else {"rtol": 1e-4, "atol": 1e-5}))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("group, keys, dim", [(9, 320, 16), (16, 512, 16), (16, 100, 64)])
+def test_one_wave_per_head_attention_of_many_heads(tmp_path, group, keys, dim):
+    """The same in float with more than 8 waves a workgroup, which take their keys in batches."""
+    from oracle import compile_cpu
+    from tests.helpers import assert_close, numpy_of
+
+    inputs = tuple(v.float() for v in attention_inputs(1, keys - 1, 2, group, dim, None))
+    exported = torch.export.export(SinkAttention(), inputs)
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        got = model(*inputs)
+    assert_close(got, compile_cpu(exported, tmp_path / "cpu")(*[numpy_of(v) for v in inputs]), rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("product", [False, True])
+@pytest.mark.parametrize("group, keys, dim", [(8, 512, 16), (9, 320, 16), (16, 320, 16), (8, 256, 32), (16, 256, 32), (8, 128, 64), (12, 128, 64), (16, 100, 64)])
+def test_one_wave_per_head_attention_fits_its_registers(tmp_path, group, keys, dim, product):
+    """A workgroup has a wave per query head: with more than 8 of them a lane's registers don't hold its keys' rows, and the
+    kernel takes them in batches: no scratch beyond what q, the sums and the batches of heads of 64 need by themselves."""
+    class Block(torch.nn.Module):
+        def forward(self, w, *operands):
+            y = SinkAttention()(*operands).reshape(1, -1)
+            return torch.nn.functional.linear(y, w) if product else y
+
+    inputs = (torch.ones(256, group * dim), *(v.float() for v in attention_inputs(1, keys - 1, 1, group, dim, None)))
+    (tmp_path / "model.hip").write_text(plan_of(Block(), *inputs))
+    remarks = subprocess.run([*compiler_command(), "-Rpass-analysis=kernel-resource-usage", str(tmp_path / "model.hip"), "-o", str(tmp_path / "out")],
+                             capture_output=True, text=True, check=True).stderr
+    names = re.findall(r"Function Name: (\S+)", remarks)
+    scratch = dict(zip(names, map(int, re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", remarks))))
+    kernels = [name for name in names if "attention" in name]
+    assert len(kernels) == 1 and product == ("attention_linear" in kernels[0]), names
+    assert scratch[kernels[0]] <= {(12, 64): 100, (16, 64): 350}.get((group, dim), 0), scratch
 
 
 @pytest.mark.gpu
