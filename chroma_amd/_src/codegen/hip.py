@@ -2229,8 +2229,8 @@ class HIPCodegen(Codegen):
         STREAM_OVERHEAD_US against ``_kwave_plan``'s, plus a launch that stores X when X is an expression. Only rows of
         STREAM_KWAVE_BYTES or more: the short rows of a vocabulary product stream faster up to 12 of them."""
         size = ITEMSIZE[x.dtype]
-        if (x.dtype not in STREAM_ROW_US or inner * size < STREAM_KWAVE_BYTES or (x.stored and not self._kwave_fits(x, weight, rows, columns, inner))
-                or inner % (16 // size) or weight.view.offset % (16 // size)):
+        stored = x if x.stored else weight  # (an expression is stored first, at the start of a buffer)
+        if x.dtype not in STREAM_ROW_US or inner * size < STREAM_KWAVE_BYTES or not self._kwave_fits(stored, weight, rows, columns, inner):
             return False
         stream = STREAM_OVERHEAD_US + columns * inner * (size / (STREAM_GBS * 1e3) + rows * STREAM_ROW_US[x.dtype] * 1e-6)
         return self._kwave_plan(rows, columns, inner, x.dtype)[0] + (0.0 if x.stored else STORE_LAUNCH_US) < stream

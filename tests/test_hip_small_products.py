@@ -50,6 +50,19 @@ def test_unaligned_operands_keep_the_general_body():
     assert "kwave_linear" not in plan_of(Function(torch.nn.functional.linear), torch.ones(40, 258), torch.ones(33, 258))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("stored", [False, True])
+def test_rows_beyond_32_bit_offsets_keep_the_general_body(dtype, stored):
+    """The K-split body's byte offsets inside a tile have 32 bits; that holds for an X that is still an expression too."""
+    from types import SimpleNamespace
+
+    x = SimpleNamespace(dtype=dtype, stored=stored, view=SimpleNamespace(offset=0) if stored else None)
+    weight = SimpleNamespace(dtype=dtype, view=SimpleNamespace(offset=0))
+    longest = 2**31 // 128 // (4 if dtype == torch.float32 else 2)
+    takes = lambda inner: HIPCodegen()._kwave_few_rows(x, weight, 8, 65536, inner)
+    assert takes(longest - 1024) and not takes(longest) and not takes(4 * longest)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows, inner, columns", [
