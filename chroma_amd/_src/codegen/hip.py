@@ -3162,9 +3162,13 @@ class HIPCodegen(Codegen):
     def _grouped_experts(self, out, weight, indices, x, tokens, selected, experts, channels, inner, per_slot) -> None:
         args = (out, weight, indices, x, tokens, selected, experts, channels, inner, per_slot)
         k, grid, threads, path, scratch = self._grouped_kernel(*args)
-        self.launch(k, grid, threads, [weight, x, scratch], kind="experts_mfma")
+        self.launch(k, grid, threads, [weight, x, scratch], kind=self._grouped_kind(path))
         self.mfma_matmuls += 1
         self.last_grouped = {"index": len(self.launches) - 1, "args": args, "path": path, "scratch": scratch}
+
+    @staticmethod
+    def _grouped_kind(path: int) -> str:
+        return "experts_kwave" if path == 4 else "experts_mfma"
 
     def _grouped_kernel(self, out, weight, indices, x, tokens, selected, experts, channels, inner, per_slot, activation=None,
                         store_product: bool = True):
@@ -3263,7 +3267,7 @@ class HIPCodegen(Codegen):
             destination, epilogue = f"static_cast<{ctype_of(out.dtype)}*>(nullptr)", ", epilogue"
         slots = min(4, KWAVE_LDS // (KWAVE_WAVES * (tm + tn) << 10))
         k.line(f"chroma::grouped_expert_kwave<{ctype_of(out.dtype)}, {str(per_slot).lower()}, {tm}, {tn}, {KWAVE_WAVES}, {slots}>({w}, {xs}, {destination}, "
-               f"reinterpret_cast<const int32_t*>({table}), {tokens * selected}u, {selected}u, {experts}u, {channels}u, {inner}u{epilogue});")
+               f"reinterpret_cast<const int32_t*>({table}), {selected}u, {experts}u, {channels}u, {inner}u{epilogue});")
         pieces = tokens * selected // (16 * tm) + experts  # at most: an expert's last piece may be partial
         return k, 8 * -(-(-(-channels // (16 * tn)) * pieces) // 8), 64 * KWAVE_WAVES, 4, scratch
 
@@ -3354,8 +3358,9 @@ class HIPCodegen(Codegen):
         except _NotFusible:
             return None
         self._retract_last_launch()
-        self.launch(k, grid, threads, [weight, xin, scratch, x], kind="experts_mfma")
-        self.product_stores.append((len(self.launches) - 1, out.root.name, lean, self.launches[-1].grid, threads, (), "experts_mfma"))
+        kind = self._grouped_kind(last["path"])
+        self.launch(k, grid, threads, [weight, xin, scratch, x], kind=kind)
+        self.product_stores.append((len(self.launches) - 1, out.root.name, lean, self.launches[-1].grid, threads, (), kind))
         self.epilogue_values[x.name] = buffer
         self.materialized[x.name] = buffer
         self.last_grouped = None

@@ -283,8 +283,8 @@ __device__ __forceinline__ ExpertPiece expert_piece_of(const int32_t* __restrict
 // ``grouped_expert_linear``; launched as 8 * ceil(ceil(C / 16 TN) * (slots / 16 TM + experts) / 8) workgroups of 64 NW threads.
 template <class T, bool PER_SLOT, int TM, int TN, int NW, int S, class Epilogue = std::nullptr_t>
 __device__ __forceinline__ void grouped_expert_kwave(const T* __restrict__ w, const T* __restrict__ x, T* __restrict__ out,
-                                                     const int32_t* __restrict__ scratch, uint32_t slots, uint32_t selected,
-                                                     uint32_t experts, uint32_t channels, uint32_t inner, Epilogue epilogue = nullptr) {
+                                                     const int32_t* __restrict__ scratch, uint32_t selected, uint32_t experts,
+                                                     uint32_t channels, uint32_t inner, Epilogue epilogue = nullptr) {
     __shared__ __attribute__((aligned(1024))) uint16_t lds[kwave_elements<TM, TN, NW, S>()];
     const int32_t* offsets = scratch + experts;
     const int32_t* permutation = scratch + 2 * experts + 2;

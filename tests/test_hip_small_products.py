@@ -193,6 +193,15 @@ def test_k_split_expert_products(tmp_path, dtype, experts, channels, inner, coun
     assert_sums(down, torch.einsum("beck,bek->bec", w, per_slot.double()), inner, 0.05, dtype)
 
 
+def test_k_split_expert_products_have_a_name_of_their_own():
+    """Profiles tell the K-split grouped products from the tiled ones by their kernels' names."""
+    weights, indices, x, per_slot = few_slots(4, 128, 128, 80)
+    names = lambda *inputs: sorted({name.rsplit("_", 1)[0] for name in re.findall(r"\bchroma_experts_\w+", plan_of(GroupedExperts(), *inputs))})
+    assert names(weights.float(), indices, x.float(), per_slot.float()) == ["chroma_experts_kwave"]
+    weights, indices, x, per_slot = few_slots(4, 384, 128, 80)
+    assert names(weights, indices, x, per_slot) == ["chroma_experts_mfma"]
+
+
 def few_slots(experts, channels, inner, slots):
     generator = torch.Generator().manual_seed(slots + channels)
     weights = (torch.randn(experts, channels, inner, generator=generator) * 0.05).bfloat16()
