@@ -2360,7 +2360,7 @@ class HIPCodegen(Codegen):
         keys = past + k_new.shape[0]
         out = self.allocate(tuple(meta.shape), meta.dtype)
         bf16 = meta.dtype == torch.bfloat16
-        if self.blas and dim in ((32, 64, 128) if bf16 else (16, 32, 64)) and self._flash_rows(tokens, kv_heads, group, keys, bf16):
+        if self.blas and dim in ((32, 64, 128) if bf16 else (16, 32, 64)) and self._flash_rows(tokens, kv_heads, group, dim, keys, bf16):
             if self._flash_attention(out, q, k_past, k_new, v_past, v_new, mask, sinks, scale):
                 return out
         if self.blas and bf16 and dim % 32 == 0 and dim <= 128 and tokens >= MATRIX_ATTENTION_TOKENS:
@@ -2406,13 +2406,20 @@ class HIPCodegen(Codegen):
         return out
 
     @staticmethod
-    def _flash_rows(tokens: int, kv_heads: int, group: int, keys: int, bf16: bool) -> bool:
+    def _flash_rows(tokens: int, kv_heads: int, group: int, dim: int, keys: int, bf16: bool) -> bool:
         """Whether an attention of these extents goes to ``attention_flash``. bfloat16: below MATRIX_ATTENTION_TOKENS queries
         every one but a decode step over a long cache (one query over more than 4 decode splits of keys has kernels of
-        its own); from there on those whose 16-query tiles would leave compute units idle and whose keys are enough
-        to split. Float: more queries than a following few-row product could take as an epilogue."""
+        its own) and short rows of one KV head over short caches, which the one-wave-per-head kernel evaluates in one batch
+        with the rotary embeddings of q and k in place and the following few-row product as its epilogue: with that product
+        8 heads of 32 over 60 / 128 / 200 keys 5.1 / 6.2 / 7.9 us against 5.8 / 5.9 / 6.1 for one query and 5.6 / 6.5 / 8.0
+        against 10.0 / 10.0 / 10.3 for 16, before q and k are stored for the latter (2 launches); 300 keys 17.5 and 7.2, and 8
+        heads of 64 over 60 keys 10.5 and 6.3. From MATRIX_ATTENTION_TOKENS queries on those whose 16-query tiles would leave
+        compute units idle and whose keys are enough to split. Float: more queries than a following few-row product could
+        take as an epilogue."""
         if not bf16:
             return tokens > 16
+        if kv_heads == 1 and tokens <= 16 and group <= 8 and dim <= 64 and group * dim <= 256 and keys <= (256 if dim <= 32 else 128):
+            return False
         if tokens < MATRIX_ATTENTION_TOKENS:
             return tokens > 1 or keys <= 4 * DECODE_SPLIT_KEYS
         return keys > 4 * DECODE_SPLIT_KEYS and kv_heads * -(-tokens // 16) < MFMA_CUS

@@ -157,6 +157,46 @@ def test_few_query_attention(tmp_path, tokens, past, kv_heads, group, dim, windo
         assert_close(result, want, rtol=2e-2, atol=1e-2)
 
 
+@pytest.mark.parametrize("tokens, keys, kv_heads, group, dim, fused", [
+    (1, 60, 1, 8, 32, True), (16, 256, 1, 8, 32, True), (4, 128, 1, 2, 64, True),
+    (17, 60, 1, 8, 32, False), (1, 257, 1, 8, 32, False), (4, 129, 1, 2, 64, False), (1, 60, 1, 8, 64, False), (1, 60, 2, 4, 32, False),
+    (1, 60, 1, 2, 128, False),
+])
+def test_short_rows_of_one_kv_head_keep_their_product(tokens, keys, kv_heads, group, dim, fused):
+    """A bfloat16 attention of one KV head over few keys and the few-row product behind it are one launch, q and k rotated in place."""
+    class Block(torch.nn.Module):
+        def forward(self, w, angle, q, k_past, k_new, *rest):
+            turn = lambda v: torch.cat((v[..., : dim // 2] * angle, v[..., dim // 2 :] * (1 - angle)), -1)
+            y = SinkAttention()(turn(q), k_past, turn(k_new), *rest)
+            return torch.nn.functional.linear(y.reshape(tokens, -1), w)
+
+    inputs = attention_inputs(tokens, keys - tokens, kv_heads, group, dim, None)
+    width = kv_heads * group * dim
+    files = lower_program(export(Block(), torch.ones(128, width, dtype=torch.bfloat16), torch.ones(1, dtype=torch.bfloat16), *inputs), HIPCodegen()).files
+    launches = [line.split()[1] for line in files["model.plan"].splitlines() if line.startswith("launch ")]
+    assert (len(launches) == 1 and "attention_linear" in launches[0]) == fused and fused != ("attention_flash<" in files["model.hip"]), launches
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens, keys, group, dim", [(1, 64, 8, 32), (5, 201, 8, 32), (16, 256, 4, 32), (3, 128, 4, 64)])
+def test_short_rows_with_their_product(tmp_path, tokens, keys, group, dim):
+    """That launch against the oracle's unfused chain at its bfloat16 bar."""
+    from oracle import compile_cpu
+    from tests.helpers import assert_close, numpy_of
+
+    class Block(torch.nn.Module):
+        def forward(self, w, *operands):
+            return torch.nn.functional.linear(SinkAttention()(*operands).reshape(tokens, -1), w)
+
+    inputs = (torch.randn(96, group * dim, generator=torch.Generator().manual_seed(keys)).to(torch.bfloat16) * 0.1,
+              *attention_inputs(tokens, keys - tokens, 1, group, dim, None))
+    exported = torch.export.export(Block(), inputs)
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        assert "stream_block_linear" in (tmp_path / "hip" / "model.hip").read_text()
+        got = model(*inputs)
+    assert_close(got, compile_cpu(exported, tmp_path / "cpu")(*[numpy_of(v) for v in inputs]), rtol=2e-2, atol=1e-2)
+
+
 class GroupedExperts(torch.nn.Module):
     def forward(self, weights, indices, x, per_slot):
         selected = weights[indices]
