@@ -113,6 +113,16 @@ STORE_LAUNCH_US = 2.5
 # The tiled bodies by the same account: (rows, columns) of a tile, and the load rate they reach when every compute unit
 # has a tile (600 x 2880 x 4096 on 128 x 192 57 us, 700 x 11520 x 2880 89 us; 2048 x 5120 x 2880 on 256 x 192 66-82 us).
 TILED_LOAD_GBS = {(256, 192): 36.0, (128, 192): 44.0}
+# ...against the K-split body, whose every round beyond the first starts with a round trip of its own, and whose float products
+# reach about 0.92 of KWAVE_MATRIX_GFLOPS (4096 x 4096 x 4096 1275 us, 2048 x 4096 x 1024 184, 20000 x 256 x 128 33).
+KWAVE_ROUND_US = {torch.float32: 1.7, torch.bfloat16: 1.5}
+KWAVE_FLOAT_SHARE = 0.92
+# Float products on the 128 x 128 body with sums in levels: this many microseconds and GFLOP/s per compute unit, whose one
+# workgroup alone takes 1.2 times as long as each of two (4096 x 4096 x 4096 1154 us, 2048 x 4096 x 1024 152, 1000 x
+# 4096 x 1024 93, 20000 x 256 x 128 24, 2048 x 5120 x 128 36 against 51 on the K-split body).
+TILED_FLOAT_OVERHEAD_US = 8.0
+TILED_FLOAT_GFLOPS = 455.0
+TILED_FLOAT_ALONE = 1.2
 # bfloat16 expert products whose channel count is a multiple of a tile width here (the first that fits)
 # take the ring body (chroma::grouped_expert_linear PATH 3) on 128-slot x width tiles with that many waves
 # side by side (each wave all slots of a width / waves strip), and an expert's last tile holds up to the
@@ -2264,20 +2274,33 @@ class HIPCodegen(Codegen):
         tiles = -(-rows // (16 * tm)) * -(-columns // (16 * tn))
         self.launch(k, 8 * -(-tiles // 8), 64 * KWAVE_WAVES, [x, weight] + ([bias] if bias is not None else []), kind="linear_kwave")
 
+    @classmethod
+    def _kwave_beats_tiles(cls, rows: int, columns: int, inner: int, dtype: torch.dtype) -> Optional[Tuple[int, int]]:
+        """The K-split body's tile where its account, with what starting each further round costs, comes out below the tiled
+        bodies'; else None."""
+        cost, tm, tn = cls._kwave_plan(rows, columns, inner, dtype)
+        rounds = -(-(-(-rows // (16 * tm)) * -(-columns // (16 * tn))) // MFMA_CUS)
+        cost += KWAVE_ROUND_US[dtype] * (rounds - 1)
+        tiled = math.inf
+        if dtype == torch.float32:
+            cost += (cost - KWAVE_OVERHEAD_US) * (1.0 / KWAVE_FLOAT_SHARE - 1.0)
+            rounds = max(TILED_FLOAT_ALONE, -(-(-(-rows // 128) * -(-columns // 128)) // MFMA_CUS))
+            tiled = TILED_FLOAT_OVERHEAD_US + rounds * 2 * 128 * 128 * inner / (TILED_FLOAT_GFLOPS * 1e3)
+        elif inner % 32 == 0:
+            tiled = min(KWAVE_OVERHEAD_US + -(-(-(-rows // m) * -(-columns // n)) // MFMA_CUS) * (m + n) * inner * 2 / (rate * 1e3)
+                        for (m, n), rate in TILED_LOAD_GBS.items())
+        return (tm, tn) if cost < tiled else None
+
     def _mfma_linear(self, out, x, weight, bias, rows, columns, inner) -> None:
-        if self._kwave_fits(x, weight, rows, columns, inner):
-            cost, tm, tn = self._kwave_plan(rows, columns, inner, out.dtype)
-            tiled = math.inf  # float products have no other body for few tiles or many
-            if out.dtype == torch.bfloat16 and inner % 32 == 0:
-                tiled = min(KWAVE_OVERHEAD_US + -(-(-(-rows // m) * -(-columns // n)) // MFMA_CUS) * (m + n) * inner * 2 / (rate * 1e3)
-                            for (m, n), rate in TILED_LOAD_GBS.items())
-            if cost < tiled:
-                # (it gains nothing from weights read ahead: 512 x 2048 x 2048 13.6 -> 15.3 us with the launch, 600 x 2880 x
-                # 4096 30.9 -> 34.6, so plans keep theirs only before small weights under many rows)
-                if rows >= KWAVE_PREFETCH[0] and columns * inner * ITEMSIZE[out.dtype] <= KWAVE_PREFETCH[1]:
-                    self._prefetch_weight(weight)
-                self._kwave_linear(out, x, weight, bias, rows, columns, inner, tm, tn)
-                return
+        fits = self._kwave_fits(x, weight, rows, columns, inner)
+        split = self._kwave_beats_tiles(rows, columns, inner, out.dtype) if fits else None
+        if split is not None:
+            # (it gains nothing from weights read ahead: 512 x 2048 x 2048 13.6 -> 15.3 us with the launch, 600 x 2880 x
+            # 4096 30.9 -> 34.6, so plans keep theirs only before small weights under many rows)
+            if rows >= KWAVE_PREFETCH[0] and columns * inner * ITEMSIZE[out.dtype] <= KWAVE_PREFETCH[1]:
+                self._prefetch_weight(weight)
+            self._kwave_linear(out, x, weight, bias, rows, columns, inner, *split)
+            return
         if not self._wide_gemm(out.dtype, inner, rows, columns):
             # (the wide body's C5 QKV product gains 3.4 us from warm weights, less than the 6.6 us read-ahead;
             # the mid body's output projection 15 us for 5.5)
@@ -2289,6 +2312,8 @@ class HIPCodegen(Codegen):
         # the 64-deep body (two workgroups per CU) when every tile fits in one round of the chip, else the
         # 32-deep body (three per CU), whose rounds quantize less
         path = 0 if tiles <= 2 * MFMA_CUS else 1
+        if fits and out.dtype == torch.float32:
+            path = 3  # sums in levels, as the K-split body's
         threads = 256
         if self._wide_gemm(out.dtype, inner, rows, columns):
             wide_tiles = -(-rows // WIDE_GEMM_TILE[0]) * -(-columns // WIDE_GEMM_TILE[1])

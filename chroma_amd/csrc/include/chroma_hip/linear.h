@@ -1239,7 +1239,11 @@ __device__ __forceinline__ void mfma_gemm_wide(const uint16_t* __restrict__ a, u
     mfma_gemm_ring<T, kWideM, kWideN, 2, 2, 5>(a, lda, b, ldb, bias, c, ldc, m_total, n_total, k_total, a_rows, c_rows, m0, n0, 1u, ring);
 }
 
-template <class T, bool B_K_CONTIGUOUS>
+// LEVELS (float): sums of 32 products, of 16 of those and of the rest, so that they are no less exact than the K-split body's
+// (kwave.h; one chain over K errs by 5.5e-7 of a result at K = 1024 and 2.0e-6 at 11520 where the K-split body's levels err by
+// 1.5e-7 and 1.9e-7). The matrix cores bound this body and the levels cost 2-5% of it: 2048 x 4096 x 1024 148 -> 152 us, 4096
+// x 4096 x 4096 1131 -> 1154; where two workgroups share a compute unit instead of three, up to 13% (1000 x 11520 x 2880).
+template <class T, bool B_K_CONTIGUOUS, bool LEVELS = false>
 __device__ __forceinline__ void mfma_gemm_sliced(const T* __restrict__ a, uint32_t lda, const T* __restrict__ b, uint32_t ldb,
                                                  const T* __restrict__ bias, T* __restrict__ c, uint32_t ldc, uint32_t m_total,
                                                  uint32_t n_total, uint32_t k_total, const int32_t* __restrict__ a_rows,
@@ -1302,6 +1306,10 @@ __device__ __forceinline__ void mfma_gemm_sliced(const T* __restrict__ a, uint32
             acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
+    f32x4_t low[LEVELS ? 4 : 1][4], high[LEVELS ? 4 : 1][4];
+    if constexpr (LEVELS) {
+        unroll<16>([&](auto t) { low[t / 4][t % 4] = high[t / 4][t % 4] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}; });
+    }
     const uint32_t steps = (k_total + BK - 1) / BK;
     fetch(0);
     stash(0);
@@ -1345,6 +1353,24 @@ __device__ __forceinline__ void mfma_gemm_sliced(const T* __restrict__ a, uint32
                 }
             }
         }
+        if constexpr (LEVELS) {
+            constexpr uint32_t LOW = 32 / BK, HIGH = 16 * LOW;
+            const bool last = step + 1 == steps;
+            if (last || step % LOW == LOW - 1) {
+                const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                unroll<16>([&](auto t) {
+                    low[t / 4][t % 4] += acc[t / 4][t % 4];
+                    acc[t / 4][t % 4] = zero;
+                });
+                if (last || step % HIGH == HIGH - 1) {
+                    unroll<16>([&](auto t) {
+                        high[t / 4][t % 4] += low[t / 4][t % 4];
+                        low[t / 4][t % 4] = zero;
+                        acc[t / 4][t % 4] = last ? high[t / 4][t % 4] : zero;
+                    });
+                }
+            }
+        }
         if (step + 1 < steps) {
             stash(buffer ^ 1);
         }
@@ -1353,8 +1379,8 @@ __device__ __forceinline__ void mfma_gemm_sliced(const T* __restrict__ a, uint32
     mfma_store<T>(acc, bias, c, ldc, m_total, n_total, c_rows, m0, n0);
 }
 
-// PATH 0 takes the 64-deep bfloat16 path whenever its conditions hold; PATH 1 always takes the sliced one;
-// PATH 2 is the direct-to-LDS body (kDirectThreads threads), for bfloat16 with a k-contiguous B, K % 64 = 0
+// PATH 0 takes the 64-deep bfloat16 path whenever its conditions hold; PATH 1 always takes the sliced one,
+// PATH 3 too, with its sums in levels (float); PATH 2 is the direct-to-LDS body (kDirectThreads threads), for bfloat16 with a k-contiguous B, K % 64 = 0
 // and lda, ldb multiples of 8, which the code generator guarantees before it selects it.
 template <class T, bool B_K_CONTIGUOUS, int PATH = 0>
 __device__ __forceinline__ void mfma_gemm(const T* __restrict__ a, uint32_t lda, const T* __restrict__ b, uint32_t ldb,
@@ -1373,7 +1399,7 @@ __device__ __forceinline__ void mfma_gemm(const T* __restrict__ a, uint32_t lda,
         }
     }
     if constexpr (PATH != 2) {
-        mfma_gemm_sliced<T, B_K_CONTIGUOUS>(a, lda, b, ldb, bias, c, ldc, m_total, n_total, k_total, a_rows, c_rows, m_base, n_base);
+        mfma_gemm_sliced<T, B_K_CONTIGUOUS, PATH == 3>(a, lda, b, ldb, bias, c, ldc, m_total, n_total, k_total, a_rows, c_rows, m_base, n_base);
     }
 }
 

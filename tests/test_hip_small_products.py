@@ -109,6 +109,38 @@ def test_k_split_float_sums(tmp_path, rows, inner, columns, levels):
     assert error < limit, (error, limit)
 
 
+@pytest.mark.parametrize("dtype, rows, columns, inner, split", [
+    (torch.float32, 800, 4096, 1024, True), (torch.float32, 700, 11520, 2880, True), (torch.float32, 2048, 1024, 4096, True),
+    (torch.float32, 2048, 4096, 1024, False), (torch.float32, 4096, 4096, 4096, False), (torch.float32, 8192, 512, 512, False),
+    (torch.float32, 20000, 256, 128, False), (torch.float32, 1024, 8192, 2048, False), (torch.float32, 2048, 5120, 128, False),
+    (torch.bfloat16, 300, 4096, 1024, True), (torch.bfloat16, 2048, 1024, 4096, True), (torch.bfloat16, 1024, 2048, 2048, True),
+    (torch.bfloat16, 4096, 1024, 1024, False), (torch.bfloat16, 1500, 2880, 2880, False), (torch.bfloat16, 20000, 256, 128, False),
+])
+def test_many_rounds_take_the_tiled_bodies(dtype, rows, columns, inner, split):
+    """Products of many tiles, each measured at least a tenth faster on the side it takes."""
+    assert (HIPCodegen._kwave_beats_tiles(rows, columns, inner, dtype) is not None) == split
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows, inner, columns", [(17, 64, 5), (129, 68, 130), (140, 520, 260), (130, 1540, 128), (64, 4096, 257)])
+def test_tiled_float_product_sums_in_levels(tmp_path, monkeypatch, rows, inner, columns):
+    """The 128 x 128 float body: one level, whole levels, ragged ones; its error against what sums of 32 products, 16 of these
+    and the rest give (``test_k_split_float_sums``)."""
+    monkeypatch.setattr(HIPCodegen, "_kwave_beats_tiles", lambda *a: None)
+    layer, x = linear(rows, inner, columns, torch.float32)
+    exported = torch.export.export(layer, (x,))
+    with chroma_amd.compile(exported, tmp_path / "hip") as model:
+        assert "mfma_linear<float, 3>" in (tmp_path / "hip" / "model.hip").read_text()
+        got = model(x)
+    exact = x.double() @ layer.weight.detach().double().T + layer.bias.detach().double()
+    assert_sums(got, exact, inner, 0.05, torch.float32)
+    error = np.linalg.norm(got - exact.numpy()) / np.linalg.norm(exact)
+    levels = (32, min(16, -(-inner // 32)), -(-inner // 512), 2)  # (the bias is one more)
+    limit = 1.2 * 0.42 * 2.0**-24 * sum((n + 1) / 2 for n in levels) ** 0.5
+    print(f"{rows} x {columns} x {inner}: {error:.3e}, limit {limit:.3e}", flush=True)
+    assert error < limit, (error, limit)
+
+
 def attention_inputs(tokens, past, kv_heads, group, dim, window):
     """Operands of a cached attention with sinks: causal (or windowed) over a cache of ``past`` rows, one query row
     wholly masked, an additive bias on a band of keys."""
