@@ -121,6 +121,20 @@ def test_many_rounds_take_the_tiled_bodies(dtype, rows, columns, inner, split):
     assert (HIPCodegen._kwave_beats_tiles(rows, columns, inner, dtype) is not None) == split
 
 
+@pytest.mark.parametrize("rows, inner, columns, split", [
+    (2, 640, 201088, False), (6, 640, 201088, False), (12, 640, 201088, True), (2, 1024, 20000, False), (8, 1024, 20000, True),
+    (2, 4096, 2880, False), (3, 4096, 2880, False), (6, 4096, 2880, True), (4, 2880, 2880, False), (6, 2880, 2880, True),
+    (2, 2880, 5120, False), (3, 2880, 5120, True), (2, 2880, 11520, False), (6, 2880, 11520, True), (8, 1024, 4096, True),
+])
+def test_few_float_rows_over_large_weights_stream(rows, inner, columns, split):
+    """Each measured at least a tenth faster on the side it takes, with weights too large for the caches."""
+    from types import SimpleNamespace
+
+    view = SimpleNamespace(offset=0)
+    x, weight = SimpleNamespace(dtype=torch.float32, stored=True, view=view), SimpleNamespace(dtype=torch.float32, view=view)
+    assert HIPCodegen()._kwave_few_rows(x, weight, rows, columns, inner) == split
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows, inner, columns", [(17, 64, 5), (129, 68, 130), (140, 520, 260), (130, 1540, 128), (64, 4096, 257)])
 def test_tiled_float_product_sums_in_levels(tmp_path, monkeypatch, rows, inner, columns):
