@@ -111,12 +111,12 @@ STREAM_ROW_US = {torch.bfloat16: 0.25, torch.float32: 0.15}
 STREAM_KWAVE_BYTES = 2 << 10
 STORE_LAUNCH_US = 2.5
 # Large float weights (from STREAM_WIDE_BYTES) are read by the K-split body at KWAVE_HBM_GBS at most, and by the stream nearly at
-# the memory's rate while X is short (STREAM_WIDE_FLOATS in all): per million elements STREAM_WIDE_US and, per row, the two of
+# the memory's rate while X is short (3 rows, or STREAM_WIDE_FLOATS in all): per million elements STREAM_WIDE_US and, per row, the two of
 # STREAM_WIDE_ROW_US, the second times K; a tenth is added, as wide as its measurements scatter. Cold weights, 2 / 3 / 4 / 6 / 8
 # rows (K-split body in parentheses): 640 -> 201088 81 / 84 / 90 / 91 / 103 (119-124), 1024 -> 20000 15 / 17 / 18 / 23 / 24 (21),
 # 4096 -> 2880 11 / 11 / 14 / 24 / 29 (16-17), 2880 -> 11520 25 / 29 / 27 / 37 / - (28-29), 2880 -> 5120 15 / 20 / 25 / 43 / - (17-18).
 STREAM_WIDE_BYTES = 30 << 20
-STREAM_WIDE_FLOATS = 16 << 10
+STREAM_WIDE_FLOATS = 8 << 10
 STREAM_WIDE_US = 0.605
 STREAM_WIDE_ROW_US = (0.033, 2.4e-5)
 KWAVE_HBM_US = 1.5
@@ -2257,7 +2257,7 @@ class HIPCodegen(Codegen):
         stream = STREAM_OVERHEAD_US + elements * (size / (STREAM_GBS * 1e3) + rows * STREAM_ROW_US[x.dtype] * 1e-6)
         if x.dtype == torch.float32 and elements * size >= STREAM_WIDE_BYTES:
             cost = max(cost, KWAVE_HBM_US + elements * size / (KWAVE_HBM_GBS * 1e3))
-            if rows * inner <= STREAM_WIDE_FLOATS:
+            if rows <= 3 or rows * inner <= STREAM_WIDE_FLOATS:
                 stream = min(stream, STREAM_OVERHEAD_US + elements * 1e-6 * (STREAM_WIDE_US + rows * (STREAM_WIDE_ROW_US[0] + STREAM_WIDE_ROW_US[1] * inner)))
         return cost + (0.0 if x.stored else STORE_LAUNCH_US) < stream
 

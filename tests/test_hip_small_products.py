@@ -123,7 +123,7 @@ def test_many_rounds_take_the_tiled_bodies(dtype, rows, columns, inner, split):
 
 @pytest.mark.parametrize("rows, inner, columns, split", [
     (2, 640, 201088, False), (6, 640, 201088, False), (12, 640, 201088, True), (2, 1024, 20000, False), (8, 1024, 20000, True),
-    (2, 4096, 2880, False), (3, 4096, 2880, False), (6, 4096, 2880, True), (4, 2880, 2880, False), (6, 2880, 2880, True),
+    (2, 4096, 2880, False), (3, 4096, 2880, False), (6, 4096, 2880, True), (6, 2880, 2880, True), (5, 2048, 8192, True),
     (2, 2880, 5120, False), (3, 2880, 5120, True), (2, 2880, 11520, False), (6, 2880, 11520, True), (8, 1024, 4096, True),
 ])
 def test_few_float_rows_over_large_weights_stream(rows, inner, columns, split):
