@@ -88,6 +88,8 @@ FLASH = [  # tokens, past, KV heads, group, dim, window
     (BF16, 40, 300, 8, 16, 64, 150),   # two row tiles
     (BF16, 33, 700, 1, 1, 64, 400),    # a group of one; split keys
     (BF16, 70, 900, 1, 8, 128, 500),
+    (BF16, 36, 4036, 8, 8, 64, 128),   # long keys, most blocks dead; split
+    (BF16, 2, 701, 8, 8, 64, 10**6),   # averages over hundreds of keys
 ]
 
 HEADS = [  # the group-shared prefill kernel: two heads a wave, one; a power-of-two scale, another
