@@ -2329,7 +2329,7 @@ class HIPCodegen(Codegen):
         # 32-deep body (three per CU), whose rounds quantize less
         path = 0 if tiles <= 2 * MFMA_CUS else 1
         if fits and out.dtype == torch.float32:
-            path = 3  # sums in levels, as the K-split body's
+            path = 5  # sums in levels, as the K-split body's
         threads = 256
         if self._wide_gemm(out.dtype, inner, rows, columns):
             wide_tiles = -(-rows // WIDE_GEMM_TILE[0]) * -(-columns // WIDE_GEMM_TILE[1])
@@ -3233,6 +3233,8 @@ class HIPCodegen(Codegen):
             threads = 64 * waves
         elif self._direct_gemm(out.dtype, inner):
             path, threads = 2, DIRECT_GEMM_THREADS
+        elif out.dtype == torch.float32 and self._kwave_fits(x, weight, tokens * selected, channels, inner):
+            path = 5  # sums in levels, as the K-split body's
         scratch, tiles = self._route(indices, experts)
         k = Kernel(1)
         if path == 3:
@@ -3282,13 +3284,19 @@ class HIPCodegen(Codegen):
         """(16-slot blocks, 16-channel blocks) of the K-split grouped body's pieces, chosen by ``_kwave_plan``'s account over
         evenly filled experts, or None: bfloat16 products keep the ring body where it applies (GPT-OSS-20B's layer of 100
         tokens 363 us on the ring, 376 here; 400 tokens 418 and 512: every piece starts with its own chain of routing
-        loads) and the direct ones above FEW_EXPERT_SLOTS slots an expert."""
+        loads) and the direct ones above FEW_EXPERT_SLOTS slots an expert, or from 16 on once their 128 x 128 tiles fill the
+        chip (32 experts of 1000 x 512: 16 slots an expert 14.4 us, 15.3 on tiles; 32 18.6 and 16.3; 62 23.0 and 17.7); float
+        ones the tiles from four rounds of the chip on (16384 slots, 8 experts of 2048 x 1024 835 us, 652 on tiles; 32 of 1024
+        x 512 249 and 226; 12 of 256 x 128, one round, 47 and 41, which the activation's own launch then costs)."""
         size = ITEMSIZE[x.dtype]
         if not self._kwave_fits(x, weight, slots, channels, inner) or channels % 4:
             return None
         if x.dtype == torch.bfloat16 and (slots > FEW_EXPERT_SLOTS * experts or inner % 32 == 0 and any(channels % n == 0 for n, _, _ in RING_EXPERT_TILES)):
             return None
         best, rows = None, -(-slots // experts)
+        tiles = experts * -(-rows // 128) * -(-channels // 128)
+        if tiles >= (MFMA_CUS if x.dtype == torch.bfloat16 else 4 * MFMA_CUS) and (x.dtype == torch.float32 or rows > 16):
+            return None
         for tm in (1, 2, 4, 8):
             for tn in (1, 2, 3, 4, 6):
                 if tm * tn > 36 or 3 * KWAVE_WAVES * (tm + tn) << 10 > KWAVE_LDS or 16 * tm >= 2 * max(16, rows):

@@ -1380,8 +1380,9 @@ __device__ __forceinline__ void mfma_gemm_sliced(const T* __restrict__ a, uint32
 }
 
 // PATH 0 takes the 64-deep bfloat16 path whenever its conditions hold; PATH 1 always takes the sliced one,
-// PATH 3 too, with its sums in levels (float); PATH 2 is the direct-to-LDS body (kDirectThreads threads), for bfloat16 with a k-contiguous B, K % 64 = 0
-// and lda, ldb multiples of 8, which the code generator guarantees before it selects it.
+// PATH 5 too, with its sums in levels (float); PATH 2 is the direct-to-LDS body (kDirectThreads threads), for
+// bfloat16 with a k-contiguous B, K % 64 = 0 and lda, ldb multiples of 8, which the code generator guarantees
+// before it selects it. (3 and 4 are bodies of expert products: grouped_expert_linear, grouped_expert_kwave.)
 template <class T, bool B_K_CONTIGUOUS, int PATH = 0>
 __device__ __forceinline__ void mfma_gemm(const T* __restrict__ a, uint32_t lda, const T* __restrict__ b, uint32_t ldb,
                                           const T* __restrict__ bias, T* __restrict__ c, uint32_t ldc, uint32_t m_total,
@@ -1399,7 +1400,7 @@ __device__ __forceinline__ void mfma_gemm(const T* __restrict__ a, uint32_t lda,
         }
     }
     if constexpr (PATH != 2) {
-        mfma_gemm_sliced<T, B_K_CONTIGUOUS, PATH == 3>(a, lda, b, ldb, bias, c, ldc, m_total, n_total, k_total, a_rows, c_rows, m_base, n_base);
+        mfma_gemm_sliced<T, B_K_CONTIGUOUS, PATH == 5>(a, lda, b, ldb, bias, c, ldc, m_total, n_total, k_total, a_rows, c_rows, m_base, n_base);
     }
 }
 

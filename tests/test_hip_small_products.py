@@ -144,7 +144,7 @@ def test_tiled_float_product_sums_in_levels(tmp_path, monkeypatch, rows, inner, 
     layer, x = linear(rows, inner, columns, torch.float32)
     exported = torch.export.export(layer, (x,))
     with chroma_amd.compile(exported, tmp_path / "hip") as model:
-        assert "mfma_linear<float, 3>" in (tmp_path / "hip" / "model.hip").read_text()
+        assert "mfma_linear<float, 5>" in (tmp_path / "hip" / "model.hip").read_text()
         got = model(x)
     exact = x.double() @ layer.weight.detach().double().T + layer.bias.detach().double()
     assert_sums(got, exact, inner, 0.05, torch.float32)
@@ -286,6 +286,42 @@ def test_k_split_expert_products_have_a_name_of_their_own():
     assert names(weights.float(), indices, x.float(), per_slot.float()) == ["chroma_experts_kwave"]
     weights, indices, x, per_slot = few_slots(4, 384, 128, 80)
     assert names(weights, indices, x, per_slot) == ["chroma_experts_mfma"]
+
+
+@pytest.mark.parametrize("dtype, experts, channels, inner, slots, split", [
+    (torch.float32, 8, 2048, 1024, 2048, True), (torch.float32, 32, 1024, 512, 4096, True), (torch.float32, 12, 256, 128, 16384, True),
+    (torch.float32, 8, 2048, 1024, 16384, False), (torch.float32, 32, 1024, 512, 16384, False),
+    (torch.bfloat16, 32, 1000, 512, 512, True), (torch.bfloat16, 8, 2048, 1024, 512, True),
+    (torch.bfloat16, 32, 1000, 512, 1024, False), (torch.bfloat16, 32, 1000, 512, 2000, False),
+])
+def test_many_expert_slots_take_the_tiled_bodies(dtype, experts, channels, inner, slots, split):
+    """Each measured faster on the side it takes."""
+    from types import SimpleNamespace
+
+    operand = SimpleNamespace(dtype=dtype, view=SimpleNamespace(offset=0))
+    assert (HIPCodegen()._kwave_experts(operand, operand, slots, experts, channels, inner) is not None) == split
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("experts, channels, inner, counts", [(3, 100, 136, [1, 63, 0]), (4, 260, 1540, [129, 0, 40, 300])])
+def test_tiled_float_expert_products(tmp_path, monkeypatch, experts, channels, inner, counts):
+    """Float expert products on 128 x 128 tiles, their sums in levels."""
+    monkeypatch.setattr(HIPCodegen, "_kwave_experts", lambda *a: None)
+    generator = torch.Generator().manual_seed(inner)
+    slots = torch.cat([torch.full((count,), e, dtype=torch.int64) for e, count in enumerate(counts)])
+    indices = slots[torch.randperm(len(slots), generator=generator)].reshape(-1, 1)
+    weights = torch.randn(experts, channels, inner, generator=generator) * 0.05
+    x, per_slot = torch.randn(len(indices), inner, generator=generator), torch.randn(*indices.shape, inner, generator=generator)
+    with chroma_amd.compile(export(GroupedExperts(), weights, indices, x, per_slot), tmp_path / "hip") as model:
+        source = (tmp_path / "hip" / "model.hip").read_text()
+        assert "grouped_expert_linear<float, false, 5" in source and "grouped_expert_linear<float, true, 5" in source
+        up, down = model(weights, indices, x, per_slot)
+    w = weights.double()[indices]
+    limit = 1.2 * 0.42 * 2.0**-24 * sum((n + 1) / 2 for n in (32, min(16, -(-inner // 32)), -(-inner // 512))) ** 0.5
+    for got, exact in ((up, torch.einsum("beck,bk->bec", w, x.double())), (down, torch.einsum("beck,bek->bec", w, per_slot.double()))):
+        assert_sums(got, exact, inner, 0.05, torch.float32)
+        error = np.linalg.norm(got - exact.numpy()) / np.linalg.norm(exact)
+        assert error < limit, (error, limit)
 
 
 def few_slots(experts, channels, inner, slots):
