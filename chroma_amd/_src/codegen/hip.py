@@ -3286,8 +3286,8 @@ class HIPCodegen(Codegen):
         tokens 363 us on the ring, 376 here; 400 tokens 418 and 512: every piece starts with its own chain of routing
         loads) and the direct ones above FEW_EXPERT_SLOTS slots an expert, or from 16 on once their 128 x 128 tiles fill the
         chip (32 experts of 1000 x 512: 16 slots an expert 14.4 us, 15.3 on tiles; 32 18.6 and 16.3; 62 23.0 and 17.7); float
-        ones the tiles from four rounds of the chip on (16384 slots, 8 experts of 2048 x 1024 835 us, 652 on tiles; 32 of 1024
-        x 512 249 and 226; 12 of 256 x 128, one round, 47 and 41, which the activation's own launch then costs)."""
+        ones the tiles from eight rounds of the chip on (16384 slots, 8 experts of 2048 x 1024: 835 us, 734 on tiles; four
+        rounds, 32 experts of 1024 x 512: 249 and 255)."""
         size = ITEMSIZE[x.dtype]
         if not self._kwave_fits(x, weight, slots, channels, inner) or channels % 4:
             return None
@@ -3295,7 +3295,7 @@ class HIPCodegen(Codegen):
             return None
         best, rows = None, -(-slots // experts)
         tiles = experts * -(-rows // 128) * -(-channels // 128)
-        if tiles >= (MFMA_CUS if x.dtype == torch.bfloat16 else 4 * MFMA_CUS) and (x.dtype == torch.float32 or rows > 16):
+        if tiles >= (MFMA_CUS if x.dtype == torch.bfloat16 else 8 * MFMA_CUS) and (x.dtype == torch.float32 or rows > 16):
             return None
         for tm in (1, 2, 4, 8):
             for tn in (1, 2, 3, 4, 6):

@@ -290,7 +290,7 @@ def test_k_split_expert_products_have_a_name_of_their_own():
 
 @pytest.mark.parametrize("dtype, experts, channels, inner, slots, split", [
     (torch.float32, 8, 2048, 1024, 2048, True), (torch.float32, 32, 1024, 512, 4096, True), (torch.float32, 12, 256, 128, 16384, True),
-    (torch.float32, 8, 2048, 1024, 16384, False), (torch.float32, 32, 1024, 512, 16384, False),
+    (torch.float32, 32, 1024, 512, 16384, True), (torch.float32, 8, 2048, 1024, 16384, False),
     (torch.bfloat16, 32, 1000, 512, 512, True), (torch.bfloat16, 8, 2048, 1024, 512, True),
     (torch.bfloat16, 32, 1000, 512, 1024, False), (torch.bfloat16, 32, 1000, 512, 2000, False),
 ])
