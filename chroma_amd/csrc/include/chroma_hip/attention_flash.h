@@ -8,12 +8,12 @@
 // global -> LDS into buffers of its own (no barrier in the loop), reads V^T fragments with the transposing LDS read,
 // and keeps (max, sum, p . v) of its keys; the waves of a workgroup meet in LDS, workgroups through ``partial`` (added
 // by ``attention_flash_combine``). What bounds it is latency: a block's copies, one round trip, behind the block before.
-// Measured on 8 KV heads of 8 heads of 64 (kernel time, before -> with the combining launch): 3 queries over 137 keys
-// 134 -> 5 us, 36 over 4072 (128-key windows) 848 -> 13, 100 over 1100 23 + 5 (live tiles) -> 9; a whole layer's call of
-// 400 queries over 2401 keys 208 -> 150 us (with its products), 480 over 4481 307 -> 220.
+// Measured back to back on 8 KV heads of 8 heads of 64 over 128-key windows, with the combining launch, against the kernels
+// that took them before: 3 queries over 137 keys 25.5 -> 4.8 us, 36 over 4072 291 -> 7.5, 100 over 1100 22.2 (with its live
+// tiles) -> 7.2.
 //
-// Float products run on v_mfma_f32_16x16x4f32 (256 queries of 8 heads of 16 over 512 keys: 25 us with a wave per query
-// head on the vector units).
+// Float products run on v_mfma_f32_16x16x4f32 (256 queries of one KV head of 8 heads of 16 over 512 keys: 8.7 us with a wave
+// per query head, 6.0 here).
 //
 // Rounding: the scores, scaled scores and masked scores are rounded as attention.h says; a probability is rounded to
 // bfloat16 as exp(s - m), m a running maximum of the row, before it meets V, and the row is divided by the float sum at

@@ -5,9 +5,10 @@
 // product over K = 2880: 40 workgroups, 45 slices). Here each of NW waves computes the whole 16 TM x 16 TN output
 // tile over its own contiguous share of K: it copies its operands global -> LDS into a ring of its own (no barrier
 // in the loop: a wave waits only for its own copies), and the waves' float partial sums meet once, in LDS, added
-// in wave order. What bounds it is the compute unit's load path, (16 TM + 16 TN) K elements per workgroup at about
-// 75 GB/s for 4 lanes to every 64-byte row piece (operand fragments read straight into registers, a lane to a row,
-// move half of that: the path is bound by the addresses of neighbouring lanes, not by bytes).
+// in wave order. What bounds it is the compute unit's load path, (16 TM + 16 TN) K elements per workgroup at 41-55 GB/s per
+// compute unit with 4 lanes to every 64-byte row piece, its first round trip included (operand fragments read straight into
+// registers, a lane to a row, move about half of that: the path is bound by the addresses of neighbouring lanes, not by
+// bytes), and for weights too large for the caches HBM at 4.3 TB/s.
 #pragma once
 
 #include "linear.h"
@@ -193,9 +194,9 @@ __device__ __forceinline__ void kwave_store(T* to, const float (&y)[4], uint32_t
 
 // A linear layer on ``kwave_tile``: 8 * ceil(tiles / 8) workgroups of 64 NW threads, the row tiles of one column tile
 // adjacent (one XCD's L2 reads each weight row once). Requires 16-byte aligned operands and rows (K a multiple of 8
-// bfloat16 or 4 float values), and X and a column tile of W below 2 GiB. Measured on cold weights, NW = 4, against
-// the 128 x 128 bodies: bfloat16 100 x 5120 x 2880 51.6 -> 18.5 us, 300 x 1024 x 4096 58.9 -> 16.0, 600 x 2880 x 4096
-// 57.3 (the 128 x 192 ring body) -> 32.9; float 256 x 160 x 128 14.3 -> 2.2, 100 x 4000 x 1000 84 -> 15.
+// bfloat16 or 4 float values), and X and a column tile of W below 2 GiB. Measured on cold weights, back to back, NW = 4, against
+// the bodies that took them before (M x N x K): bfloat16 100 x 5120 x 2880 41.4 -> 16.4 us, 100 x 2880 x 4096 52.5 -> 14.7, 300 x
+// 1024 x 4096 50.9 -> 14.6, 600 x 2880 x 4096 54.1 -> 30.4; float 256 x 160 x 128 12.2 -> 1.9, 100 x 4000 x 1000 87 -> 15.5.
 template <class T, int TM, int TN, int NW, int S, bool FINE>
 __device__ __forceinline__ void kwave_linear(const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias, T* __restrict__ out,
                                              uint32_t m_total, uint32_t n_total, uint32_t k_total) {
