@@ -128,11 +128,12 @@ TILED_LOAD_GBS = {(256, 192): 36.0, (128, 192): 44.0}
 # reach about 0.92 of KWAVE_MATRIX_GFLOPS (4096 x 4096 x 4096 1275 us, 2048 x 4096 x 1024 184, 20000 x 256 x 128 33).
 KWAVE_ROUND_US = {torch.float32: 1.7, torch.bfloat16: 1.5}
 KWAVE_FLOAT_SHARE = 0.92
-# Float products on the 128 x 128 body with sums in levels: this many microseconds and GFLOP/s per compute unit, whose one
-# workgroup alone takes 1.2 times as long as each of two (4096 x 4096 x 4096 1154 us, 2048 x 4096 x 1024 152, 1000 x
-# 4096 x 1024 93, 20000 x 256 x 128 24, 2048 x 5120 x 128 36 against 51 on the K-split body).
+# Float products on the 128 x 128 body with sums in levels: this many microseconds and GFLOP/s per compute unit (455 measured; the
+# K-split body keeps what lies within 5%), whose one workgroup alone takes 1.2 times as long as each of two (4096 x 4096 x 4096
+# 1165 us, 2048 x 4096 x 1024 154, 1000 x 4096 x 1024 94, 20000 x 256 x 128 29, 2048 x 5120 x 128 40 against 51 on the K-split body;
+# 1000 x 11520 x 2880 642 against 623).
 TILED_FLOAT_OVERHEAD_US = 8.0
-TILED_FLOAT_GFLOPS = 455.0
+TILED_FLOAT_GFLOPS = 430.0
 TILED_FLOAT_ALONE = 1.2
 # bfloat16 expert products whose channel count is a multiple of a tile width here (the first that fits)
 # take the ring body (chroma::grouped_expert_linear PATH 3) on 128-slot x width tiles with that many waves
@@ -3286,8 +3287,8 @@ class HIPCodegen(Codegen):
         tokens 363 us on the ring, 376 here; 400 tokens 418 and 512: every piece starts with its own chain of routing
         loads) and the direct ones above FEW_EXPERT_SLOTS slots an expert, or from 16 on once their 128 x 128 tiles fill the
         chip (32 experts of 1000 x 512: 16 slots an expert 14.4 us, 15.3 on tiles; 32 18.6 and 16.3; 62 23.0 and 17.7); float
-        ones the tiles from eight rounds of the chip on (16384 slots, 8 experts of 2048 x 1024: 835 us, 734 on tiles; four
-        rounds, 32 experts of 1024 x 512: 249 and 255)."""
+        ones the tiles from eight rounds of the chip on (16384 slots, 8 experts of 2048 x 1024: 835 us, 720 on tiles; four
+        rounds, 32 experts of 1024 x 512: 249 and 250)."""
         size = ITEMSIZE[x.dtype]
         if not self._kwave_fits(x, weight, slots, channels, inner) or channels % 4:
             return None

@@ -1239,10 +1239,12 @@ __device__ __forceinline__ void mfma_gemm_wide(const uint16_t* __restrict__ a, u
     mfma_gemm_ring<T, kWideM, kWideN, 2, 2, 5>(a, lda, b, ldb, bias, c, ldc, m_total, n_total, k_total, a_rows, c_rows, m0, n0, 1u, ring);
 }
 
-// LEVELS (float): sums of 32 products, of 16 of those and of the rest, so that they are no less exact than the K-split body's
-// (kwave.h; one chain over K errs by 5.5e-7 of a result at K = 1024 and 2.0e-6 at 11520 where the K-split body's levels err by
-// 1.5e-7 and 1.9e-7). The matrix cores bound this body and the levels cost 2-5% of it: 2048 x 4096 x 1024 148 -> 152 us, 4096
-// x 4096 x 4096 1131 -> 1154; where two workgroups share a compute unit instead of three, up to 13% (1000 x 11520 x 2880).
+// LEVELS (float): sums of 64 products (32 where K is below 256), of 4 of those and of the rest, the lengths of the K-split body's
+// (kwave.h), so that it errs alike: one chain over K errs by 5.5e-7 of a result at K = 1024 and 2.0e-6 at 11520, levels by 1.5e-7 and
+// 1.9e-7. The matrix cores bound this body; the levels cost their additions and a third of the workgroups a compute unit
+// holds (183 registers: two instead of three; held to three it spills and takes 4 times as long):
+// 2048 x 4096 x 1024 148 -> 154 us, 4096 x 4096 x 4096 1136 -> 1165, 20000 x 256 x 128 24 -> 29, 1000 x 11520 x 2880 567 -> 642, and 88 -> 81
+// at 65536 x 256 x 256.
 template <class T, bool B_K_CONTIGUOUS, bool LEVELS = false>
 __device__ __forceinline__ void mfma_gemm_sliced(const T* __restrict__ a, uint32_t lda, const T* __restrict__ b, uint32_t ldb,
                                                  const T* __restrict__ bias, T* __restrict__ c, uint32_t ldc, uint32_t m_total,
@@ -1354,7 +1356,7 @@ __device__ __forceinline__ void mfma_gemm_sliced(const T* __restrict__ a, uint32
             }
         }
         if constexpr (LEVELS) {
-            constexpr uint32_t LOW = 32 / BK, HIGH = 16 * LOW;
+            const uint32_t LOW = (k_total < 256u ? 32u : 64u) / BK, HIGH = 4u * LOW;  // (``k_total`` is a literal)
             const bool last = step + 1 == steps;
             if (last || step % LOW == LOW - 1) {
                 const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
