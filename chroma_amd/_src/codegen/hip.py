@@ -110,13 +110,15 @@ STREAM_GBS = 5500.0
 STREAM_ROW_US = {torch.bfloat16: 0.25, torch.float32: 0.15}
 STREAM_KWAVE_BYTES = 2 << 10
 STORE_LAUNCH_US = 2.5
-# Large float weights (from STREAM_WIDE_BYTES) are read by the K-split body at KWAVE_HBM_GBS at most, and by the stream nearly at
-# the memory's rate while X is short (3 rows, or STREAM_WIDE_FLOATS in all): per million elements STREAM_WIDE_US and, per row, the two of
-# STREAM_WIDE_ROW_US, the second times K; a tenth is added, as wide as its measurements scatter. Cold weights, 2 / 3 / 4 / 6 / 8
-# rows (K-split body in parentheses): 640 -> 201088 81 / 84 / 90 / 91 / 103 (119-124), 1024 -> 20000 15 / 17 / 18 / 23 / 24 (21),
-# 4096 -> 2880 11 / 11 / 14 / 24 / 29 (16-17), 2880 -> 11520 25 / 29 / 27 / 37 / - (28-29), 2880 -> 5120 15 / 20 / 25 / 43 / - (17-18).
-STREAM_WIDE_BYTES = 30 << 20
-STREAM_WIDE_FLOATS = 8 << 10
+# Float weights of short rows larger than the memory-side cache (STREAM_WIDE_BYTES; K up to STREAM_WIDE_INNER: a vocabulary
+# product's) are read by the K-split body at KWAVE_HBM_GBS at most, and by the stream nearly at the memory's rate: per million
+# elements STREAM_WIDE_US and, per row, the two of STREAM_WIDE_ROW_US, the second times K: 640 -> 201088 with 2 / 3 / 4 / 6 / 8 rows 81 /
+# 84 / 90 / 91 / 103 us (K-split body 119-124). Smaller weights stay with the other account: out of the cache the K-split body is as
+# quick (1024 -> 32000 with 2 / 4 rows 24 / 30 on the stream, 23), and so do longer rows: 2-4 of 2880 or 4096 values by themselves
+# stream up to a third faster from cold weights (4096 -> 2880 11 / 11 / 14 us (16)), but not behind a norm (an MLP of 3 rows, 2880 /
+# 11520, 153 us and 162 with its products streamed), and the stream's longer chains err by 2.1e-7 there against 1.7e-7.
+STREAM_WIDE_BYTES = 256 << 20
+STREAM_WIDE_INNER = 1024
 STREAM_WIDE_US = 0.605
 STREAM_WIDE_ROW_US = (0.033, 2.4e-5)
 KWAVE_HBM_US = 1.5
@@ -2256,10 +2258,9 @@ class HIPCodegen(Codegen):
             return False
         cost, elements = self._kwave_plan(rows, columns, inner, x.dtype)[0], columns * inner
         stream = STREAM_OVERHEAD_US + elements * (size / (STREAM_GBS * 1e3) + rows * STREAM_ROW_US[x.dtype] * 1e-6)
-        if x.dtype == torch.float32 and elements * size >= STREAM_WIDE_BYTES:
+        if x.dtype == torch.float32 and elements * size >= STREAM_WIDE_BYTES and inner <= STREAM_WIDE_INNER:
             cost = max(cost, KWAVE_HBM_US + elements * size / (KWAVE_HBM_GBS * 1e3))
-            if rows <= 3 or rows * inner <= STREAM_WIDE_FLOATS:
-                stream = min(stream, STREAM_OVERHEAD_US + elements * 1e-6 * (STREAM_WIDE_US + rows * (STREAM_WIDE_ROW_US[0] + STREAM_WIDE_ROW_US[1] * inner)))
+            stream = min(stream, STREAM_OVERHEAD_US + elements * 1e-6 * (STREAM_WIDE_US + rows * (STREAM_WIDE_ROW_US[0] + STREAM_WIDE_ROW_US[1] * inner)))
         return cost + (0.0 if x.stored else STORE_LAUNCH_US) < stream
 
     @staticmethod

@@ -122,12 +122,11 @@ def test_many_rounds_take_the_tiled_bodies(dtype, rows, columns, inner, split):
 
 
 @pytest.mark.parametrize("rows, inner, columns, split", [
-    (2, 640, 201088, False), (6, 640, 201088, False), (12, 640, 201088, True), (2, 1024, 20000, False), (8, 1024, 20000, True),
-    (2, 4096, 2880, False), (3, 4096, 2880, False), (6, 4096, 2880, True), (6, 2880, 2880, True), (5, 2048, 8192, True),
-    (2, 2880, 5120, False), (3, 2880, 5120, True), (2, 2880, 11520, False), (6, 2880, 11520, True), (8, 1024, 4096, True),
+    (2, 640, 201088, False), (6, 640, 201088, False), (12, 640, 201088, True), (4, 1024, 32000, True), (8, 1024, 4096, True),
+    (3, 2880, 11520, True), (3, 11520, 2880, True), (4, 2048, 8192, True),
 ])
 def test_few_float_rows_over_large_weights_stream(rows, inner, columns, split):
-    """Each measured at least a tenth faster on the side it takes, with weights too large for the caches."""
+    """Each measured faster on the side it takes, (the last three behind an MLP's norm)."""
     from types import SimpleNamespace
 
     view = SimpleNamespace(offset=0)
