@@ -126,7 +126,7 @@ def test_many_rounds_take_the_tiled_bodies(dtype, rows, columns, inner, split):
     (3, 2880, 11520, True), (3, 11520, 2880, True), (4, 2048, 8192, True),
 ])
 def test_few_float_rows_over_large_weights_stream(rows, inner, columns, split):
-    """Each measured faster on the side it takes, (the last three behind an MLP's norm)."""
+    """Each measured faster on the side it takes (the last three behind an MLP's norm)."""
     from types import SimpleNamespace
 
     view = SimpleNamespace(offset=0)
